@@ -10,12 +10,12 @@
 //  * keys are walked in 32-key tiles.  k_pf_image first dequantises every tile of the call's KV range once into an
 //    fp16 image (K as [key][dim], V transposed as [dim][key], XOR-swizzled 16-byte units), so both MFMA A-operands
 //    are single conflict-free 16-byte LDS reads; k_prefill copies the images HBM -> LDS by direct-to-LDS loads (no
-//    registers) two tiles ahead, one barrier per tile.  Built with QWA_PF_IMAGE=0, the raw quantized bytes go to
+//    registers) two tiles ahead, one barrier per tile.  In short passes (pf_use_image) the raw quantized bytes go to
 //    LDS instead and all threads dequantise the next tile cooperatively inside the loop;
 //  * S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_16x16x32_f16 (fp32 accumulation); P^T comes out of the S^T
 //    accumulator already in B-operand layout; online softmax in fp32 with a lazy rescale;
 //  * the causal key range of a row block is cut into fixed splits (pf_splits) so that the 24 row blocks x 4 KV
-//    heads of a 1024-token chunk fill the chip; the (row block, KV head, split) units run one per workgroup, or, for
+//    heads of a 1024-token chunk fill the chip, up to 64 of them for the one row block of a short chunk; the (row block, KV head, split) units run one per workgroup, or, for
 //    a 1024-token pass, three consecutive ones per workgroup in a single round (pf_units_per_wg), a run of splits of
 //    one row block being walked as one key range.  Each run leaves a partial state (m, l, O / l) in the caller's
 //    workspace and k_pf_combine merges them in a fixed order, applies the sigmoid gate and writes fp16.  Chunks
@@ -46,20 +46,39 @@ constexpr int PF_TILE = 32;                      // keys per tile
 constexpr int PF_KT = PF_TILE / 16;              // 16-key MFMA tiles per tile
 constexpr int PF_NS = PF_ROWS == 192 ? 6 : 8;    // key-range splits per row block (3 rounds of the chip for B = 1024)
 constexpr int PF_MAXB = 1024;                    // tokens per pass
-#ifndef QWA_PF_FILL
-#define QWA_PF_FILL 1
-#endif
-// splits of a pass of nb tokens (at most PF_NS): the count that fills the chip's 256 CUs in whole rounds best, i.e.
-// the fewest rounds per split, ceil(workgroups / 256) / splits (1024 tokens: 8 splits, 3 rounds; 512 tokens: 5
-// splits, one round of 240 workgroups, where 8 would make 1.5 rounds)
-inline int pf_splits(int nb) {
-    if (!QWA_PF_FILL) return PF_NS;
-    const int groups = (GRP * nb + PF_ROWS - 1) / PF_ROWS * NKV;
+// row blocks of a pass of nb tokens (per KV head)
+inline int pf_row_blocks(int nb) { return (GRP * nb + PF_ROWS - 1) / PF_ROWS; }
+constexpr int PF_FEW = 12;  // row blocks up to which a pass takes the split count that fills one round of the chip
+// splits of a pass of nb tokens whose keys end at npos.
+// Up to PF_FEW row blocks (512 tokens): as many as make one round of the 256 CUs (64 / row blocks per KV head), each of
+// at least one tile.  (Fewer splits for short key ranges, sqrt(c tiles / tokens) with c = 500 .. 2000 to weigh the
+// partial states, measured the same or up to 3 us slower at contexts below 4000.)
+// Measured, whole call, us, against 5 to 8 splits for every pass (Q8_0): 8 tokens at 20000 positions 153 -> 48, 77 at
+// 20011 167 -> 84, 77 at 90000 648 -> 281, 128 at 32256 255 -> 152, 200 at 5000 69 -> 60, 256 at 32256 261 -> 235;
+// 512 tokens unchanged (their 5 splits already make one round).
+// Above that (at most PF_NS): the count that fills the chip's 256 CUs in whole rounds best, i.e. the fewest rounds per
+// split, ceil(workgroups / 256) / splits (1024 tokens: 8 splits, 3 rounds).
+inline int pf_splits(int nb, int npos) {
+    const int nrb = pf_row_blocks(nb);
+    if (nrb <= PF_FEW) return min(256 / (NKV * nrb), (npos - 1) / PF_TILE + 1);
+    const int groups = nrb * NKV;
     int best = PF_NS;
     for (int ns = PF_NS - 1; ns >= 5; ns--)  // 5 .. PF_NS: the instantiated kernels
         if ((long)((groups * ns + 255) / 256) * best < (long)((groups * best + 255) / 256) * ns) best = ns;
     return best;
 }
+// Whether a call dequantises its KV range into fp16 images first.  The image pass and the wider fp16 stream pay when
+// several row blocks read a tile; up to these counts every workgroup converts its raw tiles in the loop instead.
+// Whole call, us, images / raw tiles: F16 42 tokens at 60000 positions 166 / 100, 77 at 20011 92 / 76, 170 at 20000
+// (4 blocks) 127 / 122, 256 at 32256 (6) 243 / 253; Q4_0 150 / 105, 84 / 80, 120 / 128 (4 blocks); Q8_0 150 / 129,
+// 84 / 88, 122 / 144.
+inline bool pf_use_image(int kvt, int nb) {
+    return pf_row_blocks(nb) > (kvt == QWA_KV_F16 ? 4 : kvt == QWA_KV_Q4_0 ? 2 : 1);
+}
+// token-splits (splits x tokens) that a workspace for passes of up to nb tokens has to hold: PF_NS per token, or what
+// the shorter passes take (at most 256 / NKV / row blocks splits each: 2736 token-splits cover every count of row
+// blocks), never decreasing in nb
+inline int pf_token_splits(int nb) { return max(PF_NS * nb, min(256 / NKV * nb, 2736)); }
 #ifndef QWA_PF_UPW
 #define QWA_PF_UPW 1
 #endif
@@ -74,9 +93,9 @@ inline int pf_splits(int nb) {
 // ~80000 positions a workgroup's three splits are long enough for the row blocks sharing an XCD's L2 to drift apart.
 // (QWA_PF_UPW = 0: always rounds.)
 inline int pf_units_per_wg(int nb, int npos) {
-    const int ns = pf_splits(nb);
-    if (!QWA_PF_UPW || ns != 8 || npos > QWA_PF_SEG_MAXPOS) return 1;
-    const int units = (GRP * nb + PF_ROWS - 1) / PF_ROWS * NKV * ns;
+    const int nrb = pf_row_blocks(nb), ns = pf_splits(nb, npos);
+    if (!QWA_PF_UPW || nrb <= PF_FEW || ns != 8 || npos > QWA_PF_SEG_MAXPOS) return 1;
+    const int units = nrb * NKV * ns;
     return (units + 255) / 256;
 }
 constexpr int KS_LD = HD + 8;                    // K tile row stride (halves)
@@ -272,11 +291,6 @@ __device__ __forceinline__ void pf_convert(const uint8_t* raw, _Float16* Ks, _Fl
     }
 }
 
-#ifndef QWA_PF_IMAGE
-#define QWA_PF_IMAGE 1
-#endif
-// fp16 tile images: the KV range is dequantised once per call (k_pf_image), not once per row block inside the loop
-constexpr bool PF_IMAGE = QWA_PF_IMAGE != 0;
 constexpr int PF_IMG_K = PF_TILE * HD * 2;      // bytes of the K part of an image: [32 keys][256 dims] fp16
 constexpr int PF_IMG_BYTES = 2 * PF_IMG_K;      // K part, then V^T part [256 dims][32 keys] fp16
 constexpr int PF_IMG_NBUF = 3;   // images in LDS: the one computed on and two in flight
@@ -370,11 +384,14 @@ using PfPartMl = float4;  // (m, l, scale, unused)
 // p0 .. p0 + B - 1.
 // IMG: tiles come as fp16 images (k_pf_image) of img_tiles tiles per KV head, copied straight into LDS; otherwise as
 // raw quantized bytes dequantised in the loop.
+// NS: the split count; 0: ns_rt splits, and the waves whose rows all lie past the last one only load and wait (a short
+// pass fills its last row block badly).
 template <int KVT, bool IMG, int NS>
 __global__ void __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(PF_WPE, PF_WPE)))
 k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uint8_t* __restrict__ img, int img_tiles,
-          PfPartO* __restrict__ part_o, PfPartMl* __restrict__ part_ml, int ps, int upw, unsigned long long* prof) {
+          PfPartO* __restrict__ part_o, PfPartMl* __restrict__ part_ml, int ps, int upw, int ns_rt, unsigned long long* prof) {
     prof_start(prof);
+    const int ns = NS ? NS : ns_rt;
     using L = PfRaw<KVT>;
     constexpr int NBUF = IMG ? PF_IMG_NBUF : L::NBUF;
     constexpr int AHEAD = IMG ? PF_IMG_AHEAD : NBUF - 1;
@@ -390,7 +407,7 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
     // workgroups that one XCD runs (w = x mod 8) then all start at split (upw x) mod NS and move through the splits in
     // step, so they read the same image tiles at the same time, as the XCD-aware numbering of upw = 1 arranges.
     const int nrb = (GRP * B + PF_ROWS - 1) / PF_ROWS;
-    const int units = nrb * NKV * NS;
+    const int units = nrb * NKV * ns;
     int unit = upw == 1 ? 0 : (int)blockIdx.x * upw;
     const int unit_end = upw == 1 ? 1 : min(unit + upw, units);
     for (int seg = 0; unit < unit_end; seg++) {
@@ -403,10 +420,10 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
             bx = blockIdx.x;
             g = blockIdx.y;
             sp = blockIdx.z;
-            if constexpr ((NKV * NS) % 8 == 0) {
+            if ((NKV * ns) % 8 == 0) {
                 const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
                 const int xcd = lin & 7, slot = lin >> 3;
-                const int pair = NKV * NS / 8 * xcd + slot / nrb;
+                const int pair = NKV * ns / 8 * xcd + slot / nrb;
                 bx = slot % nrb;
                 g = pair % NKV;
                 sp = pair / NKV;
@@ -419,9 +436,9 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
             sp_last = sp;
             unit = 1;
         } else {
-            const int pr = unit / NS;
-            sp = unit % NS;
-            sp_last = min(NS - 1, sp + (unit_end - unit) - 1);
+            const int pr = unit / ns;
+            sp = unit % ns;
+            sp_last = min(ns - 1, sp + (unit_end - unit) - 1);
             g = pr / nrb;
             bx = pr % nrb;
             unit += sp_last - sp + 1;
@@ -433,7 +450,7 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
         const int last_row = min(row0 + PF_ROWS, nrows) - 1;
         const int kmax = p0 + last_row / GRP;
         const int n_tiles = kmax / PF_TILE + 1;
-        const int tb = sp * n_tiles / NS, nt = (sp_last + 1) * n_tiles / NS - tb;
+        const int tb = sp * n_tiles / ns, nt = (sp_last + 1) * n_tiles / ns - tb;
         const size_t rowbase = (size_t)g * kv.capacity;
         const int nvm = IMG ? PF_IMG_BYTES / 1024 / PF_WAVES : L::count(wave);
         uint32_t raw_lds[NBUF];
@@ -519,6 +536,11 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
         };
         for (int i = 0; i < nt; i++) {
             const int k0 = (tb + i) * PF_TILE, cur = i & 1;
+            // raw Q4_0 tiles: opaque copies of the thread index, so that the load's and the conversion's per-thread
+            // addresses are formed anew for every tile instead of living across the loop (31 -> 18 spilled registers;
+            // 42 tokens at 60000 positions 112 -> 105 us; the other formats measured 1-5% slower this way)
+            int tl = t, ll = lane;
+            if constexpr (!IMG && KVT == QWA_KV_Q4_0) asm volatile("" : "+v"(tl), "+v"(ll));
             // tile i + AHEAD (the last tile again near the end: a harmless re-read) into the raw buffer freed last
             // iteration
             if constexpr (IMG)
@@ -526,14 +548,14 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
                              wave, lane);
             else
                 pf_issue<KVT>(raw_lds[(i + AHEAD) % NBUF], kv, rowbase, (tb + min(i + AHEAD, nt - 1)) * PF_TILE, kmax,
-                              wave, lane);
+                              wave, ll);
             const _Float16* Ks = IMG ? reinterpret_cast<const _Float16*>(s_raw[i % NBUF]) : s_k[cur];
             const _Float16* Vt = IMG ? Ks + PF_IMG_K / 2 : s_vt[cur];
 
             // the next tile's raw bytes landed before the last barrier: dequantise them into the other fp16 tile
             auto convert = [&]() {
                 if constexpr (!IMG && AHEAD >= 2)
-                    pf_convert<KVT>(s_raw[(i + 1) % NBUF], s_k[cur ^ 1], s_vt[cur ^ 1], t);
+                    pf_convert<KVT>(s_raw[(i + 1) % NBUF], s_k[cur ^ 1], s_vt[cur ^ 1], tl);
             };
 
             f4 sc[PF_RT][PF_KT];
@@ -634,9 +656,11 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
             };
 
             if (!IMG && lead) convert();
-            scores();
-            softmax();
-            pv(Vt);
+            if (NS != 0 || wrow0 < nrows) {
+                scores();
+                softmax();
+                pv(Vt);
+            }
             if (!IMG && !lead) convert();
 
             if constexpr (IMG) {
@@ -650,7 +674,7 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
             } else {
                 wait_vm(0);
                 __syncthreads();
-                if (i + 1 < nt) pf_convert<KVT>(s_raw[(i + 1) % L::NBUF], s_k[cur ^ 1], s_vt[cur ^ 1], t);
+                if (i + 1 < nt) pf_convert<KVT>(s_raw[(i + 1) % L::NBUF], s_k[cur ^ 1], s_vt[cur ^ 1], tl);
                 __syncthreads();
             }
         }
@@ -726,14 +750,56 @@ __global__ void __launch_bounds__(256) k_pf_combine(const float* __restrict__ ga
         make_uint2((uint32_t)h0 | ((uint32_t)h1 << 16), (uint32_t)h2v | ((uint32_t)h3 << 16));
 }
 
-// Workspace layout of one call: the fp16 images of the KV range [0, p0 + B) (NKV x tiles x 32 KB; none when built
-// without images), then the (m, l) pairs and the partial O of one pass (up to PF_NS x ps rows, ps = NH x min(B,
-// PF_MAXB)).
+// The same merge for any split count up to 64 (passes of few row blocks): lane s holds split s's (m, l, scale), the
+// weights are wave reductions, and the partial rows are read eight splits at a time.
+__global__ void __launch_bounds__(256) k_pf_combine_any(const float* __restrict__ gate, int nrows, int ns,
+                                                        const PfPartO* __restrict__ part_o,
+                                                        const PfPartMl* __restrict__ part_ml, int ps,
+                                                        uint16_t* __restrict__ out16) {
+    const int rr = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (rr >= nrows) return;
+    const float4 gv = *reinterpret_cast<const float4*>(gate + (size_t)rr * HD + 4 * lane);
+    const PfPartMl ml = lane < ns ? part_ml[(size_t)lane * ps + rr] : make_float4(-INFINITY, 0.0f, 0.0f, 0.0f);
+    const PfPartO* po = part_o + (size_t)rr * (HD / 4) + lane;
+    constexpr int U = 8;
+    PfPartO ov[U];
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int u = 0; u < U; u++) ov[u] = po[(size_t)min(u, ns - 1) * ps * (HD / 4)];
+    const float mx = wave_max(ml.x);
+    const float w = ml.x == -INFINITY ? 0.0f : fast_exp2((ml.x - mx) * PF_LOG2E) * ml.y;
+    const float wq = w * ml.z, wsum = wave_sum(w);  // wq = 0 in the lanes past ns: those re-read a split's row
+    for (int s0 = 0; s0 < ns; s0 += U) {
+        PfPartO nx[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) nx[u] = po[(size_t)min(s0 + U + u, ns - 1) * ps * (HD / 4)];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wq), min(s0 + u, 63)));
+            const float4 v = unpack16x4(ov[u]);
+            const float fs = s0 + u < ns ? f : 0.0f;
+            acc.x = fmaf(fs, v.x, acc.x);
+            acc.y = fmaf(fs, v.y, acc.y);
+            acc.z = fmaf(fs, v.z, acc.z);
+            acc.w = fmaf(fs, v.w, acc.w);
+            ov[u] = nx[u];
+        }
+    }
+    const float iw = 1.0f / wsum;
+    const uint16_t h0 = f2h_bits(acc.x * iw * sigmoid(gv.x)), h1 = f2h_bits(acc.y * iw * sigmoid(gv.y));
+    const uint16_t h2v = f2h_bits(acc.z * iw * sigmoid(gv.z)), h3 = f2h_bits(acc.w * iw * sigmoid(gv.w));
+    *reinterpret_cast<uint2*>(out16 + (size_t)rr * HD + 4 * lane) =
+        make_uint2((uint32_t)h0 | ((uint32_t)h1 << 16), (uint32_t)h2v | ((uint32_t)h3 << 16));
+}
+
+// Workspace layout of one call: the fp16 images of the KV range [0, p0 + B) (NKV x tiles x 32 KB; unused by
+// calls that convert in the loop), then the (m, l) pairs and the partial O of one pass (NH rows per token-split,
+// pf_token_splits).
 struct PfWork {
     uint8_t* img;
     PfPartMl* ml;
     PfPartO* o;  // 4 values per element
-    int tiles, ps;
+    int tiles;
     size_t bytes;
 };
 
@@ -742,10 +808,10 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 static PfWork pf_work_layout(uint8_t* base, int B, int n_pos) {
     PfWork w;
     w.tiles = (n_pos - 1) / PF_TILE + 1;
-    w.ps = NH * min(B, PF_MAXB);
-    const size_t img = PF_IMAGE ? align256((size_t)NKV * w.tiles * PF_IMG_BYTES) : 0;
-    const size_t ml = align256((size_t)PF_NS * w.ps * sizeof(PfPartMl));
-    const size_t o = (size_t)PF_NS * w.ps * (HD / 4) * sizeof(PfPartO);
+    const size_t rows = (size_t)NH * pf_token_splits(min(B, PF_MAXB));
+    const size_t img = align256((size_t)NKV * w.tiles * PF_IMG_BYTES);
+    const size_t ml = align256(rows * sizeof(PfPartMl));
+    const size_t o = rows * (HD / 4) * sizeof(PfPartO);
     w.img = base;
     w.ml = reinterpret_cast<PfPartMl*>(base + img);
     w.o = reinterpret_cast<PfPartO*>(base + img + ml);
@@ -755,28 +821,34 @@ static PfWork pf_work_layout(uint8_t* base, int B, int n_pos) {
 
 size_t prefill_work_bytes(int B, int n_pos) { return pf_work_layout(nullptr, B, n_pos).bytes; }
 
-template <int KVT>
+template <int KVT, bool IMG>
 static void launch_prefill_pass(const float* qp, const qwa_kv_layer& kv, int nb, int p0, const PfWork& w,
                                 hipStream_t st) {
-    const int ns = pf_splits(nb);
+    const int ns = pf_splits(nb, p0 + nb);
     const int upw = pf_units_per_wg(nb, p0 + nb);
-    const int nrb = (GRP * nb + PF_ROWS - 1) / PF_ROWS, units = nrb * NKV * ns;
+    const int nrb = pf_row_blocks(nb), units = nrb * NKV * ns;
     const dim3 grid = upw == 1 ? dim3(nrb, NKV, ns) : dim3((units + upw - 1) / upw);
     const ProfSlot ps = profile_slot(grid.x * grid.y * grid.z, st);
 #define QWA_PF_LAUNCH(N)                                                                                              \
-    QWA_LAUNCH_MAIN(ps, (k_prefill<KVT, PF_IMAGE, N>), grid, dim3(PF_THREADS), st, qp, kv, nb, p0, w.img, w.tiles, \
-                    w.o, w.ml, w.ps, upw)
-    if (ns == 5) QWA_PF_LAUNCH(5);
-    else if (ns == 6) QWA_PF_LAUNCH(6);
-    else if (ns == 7) QWA_PF_LAUNCH(7);
-    else QWA_PF_LAUNCH(PF_NS);
+    QWA_LAUNCH_MAIN(ps, (k_prefill<KVT, IMG, N>), grid, dim3(PF_THREADS), st, qp, kv, nb, p0, w.img, w.tiles, \
+                    w.o, w.ml, NH * nb, upw, ns)
+    if constexpr (IMG) {
+        if (nrb <= PF_FEW) QWA_PF_LAUNCH(0);
+        else if (ns == 5) QWA_PF_LAUNCH(5);
+        else if (ns == 6) QWA_PF_LAUNCH(6);
+        else if (ns == 7) QWA_PF_LAUNCH(7);
+        else QWA_PF_LAUNCH(PF_NS);
+    } else {
+        QWA_PF_LAUNCH(0);
+    }
 #undef QWA_PF_LAUNCH
 }
 
 hipError_t launch_prefill(const float* q, const float* gate, const qwa_kv_layer& kv, int kvt, int B, int p0,
                           uint16_t* out16, void* work, hipStream_t st) {
     const PfWork w = pf_work_layout(static_cast<uint8_t*>(work), B, p0 + B);
-    if (PF_IMAGE) {
+    const bool image = pf_use_image(kvt, min(B, PF_MAXB));
+    if (image) {
         const dim3 grid(w.tiles, NKV);
         if (kvt == QWA_KV_F16)
             hipLaunchKernelGGL(k_pf_image<QWA_KV_F16>, grid, dim3(PF_THREADS), 0, st, kv, p0 + B - 1, w.tiles, w.img);
@@ -788,19 +860,31 @@ hipError_t launch_prefill(const float* q, const float* gate, const qwa_kv_layer&
     for (int t0 = 0; t0 < B; t0 += PF_MAXB) {
         const int nb = min(PF_MAXB, B - t0);
         const float* qp = q + (size_t)t0 * NH * HD;
-        if (kvt == QWA_KV_F16) launch_prefill_pass<QWA_KV_F16>(qp, kv, nb, p0 + t0, w, st);
-        else if (kvt == QWA_KV_Q8_0) launch_prefill_pass<QWA_KV_Q8_0>(qp, kv, nb, p0 + t0, w, st);
-        else launch_prefill_pass<QWA_KV_Q4_0>(qp, kv, nb, p0 + t0, w, st);
+#define QWA_PF_PASS(T)                                                              \
+    case T:                                                                         \
+        if (image) launch_prefill_pass<T, true>(qp, kv, nb, p0 + t0, w, st);        \
+        else launch_prefill_pass<T, false>(qp, kv, nb, p0 + t0, w, st);             \
+        break
+        switch (kvt) {
+            QWA_PF_PASS(QWA_KV_F16);
+            QWA_PF_PASS(QWA_KV_Q8_0);
+            default: QWA_PF_PASS(QWA_KV_Q4_0);
+        }
+#undef QWA_PF_PASS
         const int nrows = nb * NH;
         const float* gp = gate + (size_t)t0 * NH * HD;
         uint16_t* op = out16 + (size_t)t0 * NH * HD;
         const dim3 cg((nrows + 3) / 4), cb(256);
-        const int upw = pf_units_per_wg(nb, p0 + t0 + nb);
-        switch (pf_splits(nb)) {
+        const int upw = pf_units_per_wg(nb, p0 + t0 + nb), ns = pf_splits(nb, p0 + t0 + nb);
+        if (pf_row_blocks(nb) <= PF_FEW) {
+            hipLaunchKernelGGL(k_pf_combine_any, cg, cb, 0, st, gp, nrows, ns, w.o, w.ml, nrows, op);
+            continue;
+        }
+        switch (ns) {
 #define QWA_PF_COMBINE(N) \
-    case N: hipLaunchKernelGGL(k_pf_combine<N>, cg, cb, 0, st, gp, nrows, w.o, w.ml, w.ps, upw, op); break
+    case N: hipLaunchKernelGGL(k_pf_combine<N>, cg, cb, 0, st, gp, nrows, w.o, w.ml, nrows, upw, op); break
             QWA_PF_COMBINE(5); QWA_PF_COMBINE(6); QWA_PF_COMBINE(7);
-            default: hipLaunchKernelGGL(k_pf_combine<PF_NS>, cg, cb, 0, st, gp, nrows, w.o, w.ml, w.ps, upw, op); break;
+            default: hipLaunchKernelGGL(k_pf_combine<PF_NS>, cg, cb, 0, st, gp, nrows, w.o, w.ml, nrows, upw, op); break;
 #undef QWA_PF_COMBINE
         }
     }

@@ -2,7 +2,7 @@
 against the FP32 test kernel at the reference's chunk cases (tests/kernels/test_attn_prefill.cu:20-72: a cache of
 1500 positions filled through rope_table + attn_prep_rows, chunks (p0, B) in {(0,37), (0,512), (300,129),
 (1000,500), (1480,20)}), plus a 1300-token chunk (two passes of the kernel's 1024-token limit), chunks of 420 and 360
-tokens (the kernel cuts their key ranges into 6 and 7 splits; 500 and 512 take 5, the rest 8), long-context chunks
+tokens (key ranges cut into other split counts), long-context chunks
 of every format, the BASELINE 1024-token chunk at p0 = 32768 on all of its queries, and the ownership contract of
 the workspace: the caller-owned form gives the drop-in call's bits, a captured HIP graph replays correctly, two
 streams with their own workspaces do not interfere, a stream without a reservation gets one on first use (outside
@@ -321,7 +321,7 @@ def test_prefill_at_max_positions(gpu, oracle):
 
 @pytest.mark.parametrize("kvt", KVTS, ids=lambda k: KV_NAMES[k])
 def test_prefill_random_sweep(gpu, oracle, kvt):
-    """Seeded random chunks (p0, B) over one cache of 20000 positions, B in 1..1400 (one or two passes, 5 to 8 splits,
+    """Seeded random chunks (p0, B) over one cache of 20000 positions, B in 1..1400 (one or two passes, any split count,
     units grouped per workgroup or not): every row against the FP32 test kernel (the reference's bound), the first and
     last 8 rows against the oracle."""
     n_pos = 20000
