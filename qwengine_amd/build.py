@@ -19,7 +19,7 @@ LIB = os.path.join(OUT_DIR, "libqwattn.so")
 ARCH = "gfx950"
 
 SOURCES = ["capi.hip", "kv_append.hip", "attn_decode.hip", "attn_decode_ilp.hip", "attn_simple.hip", "attn_prefill.hip",
-           "deltanet.hip", "gemv.hip", "gemv_mc.hip", "gemm.cpp"]
+           "deltanet.hip", "deltanet_rows.hip", "gemv.hip", "gemv_mc.hip", "gemm.cpp"]
 
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
@@ -53,6 +53,7 @@ ILP_SCHED = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
 FILE_FLAGS = {"attn_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "attn_decode_ilp.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", *ILP_SCHED],
               "deltanet.hip": ILP_SCHED,
+              "deltanet_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               # gemv_mc.hip (IQ4_XS / IQ2_S one-column GEMV): the max-memory-clause scheduler
               "gemv_mc.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"]}
 
