@@ -680,12 +680,23 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
         }
         wait_vmcnt<0>();  // no direct-to-LDS load outlives the workgroup
 
-        // ---- partial state of this split: (m, l) and O / l; lane holds dims 16 dt + 4 lg + i of row (rt, i16)
+        // ---- partial state of this split: (m, l) and O / l; lane holds dims 16 dt + 4 lg + i of row (rt, i16).  A lane's
+        // 8 bytes per dim tile change lanes in the ring's LDS (8 KB per wave and row tile, XOR-swizzled 8-byte units), so
+        // that a store instruction writes two whole 512-byte rows instead of 32-byte pieces of 16 rows.  Whole call, us:
+        // 509 tokens at 0 F16 39.7 -> 36.2, 77 at 20011 Q8_0 87.7 -> 82.7, 256 at 32256 242.8 -> 240.1; the 1024-token
+        // kernel (8 splits), whose one store per 400 tiles does not matter, measured 774 -> 778 and stores directly, as do
+        // the raw-tile kernels, whose ring is too small
+        constexpr bool VIA_LDS = IMG && NS != 8;
+        // (an opaque copy of the lane: the addresses below must not live across the key loop)
+        int el = lane;
+        if constexpr (VIA_LDS) asm volatile("" : "+v"(el));
+        const int ei = VIA_LDS ? el & 15 : i16, eg = VIA_LDS ? el >> 4 : lg;
+        uint2* const xch = reinterpret_cast<uint2*>(&s_raw[0][0]) + wave * 1024;
+        if constexpr (VIA_LDS) __syncthreads();  // no wave's images are in flight any more
 #pragma unroll
         for (int rt = 0; rt < PF_RT; rt++) {
             const float lt = rows_sum(l[rt]);
-            if (qpos[rt] < 0) continue;
-            const int r = wrow0 + 16 * rt + i16, rr = (r / GRP) * NH + g * GRP + r % GRP;
+            const int r = wrow0 + 16 * rt + ei, rr = (r / GRP) * NH + g * GRP + r % GRP;
             const size_t prow = (size_t)sp * ps + rr;
             const float il = lt > 0.0f ? 1.0f / lt : 0.0f;  // a split that saw no key leaves l = 0 and O = 0
             float amax = 0.0f;
@@ -696,11 +707,30 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
             amax = rows_max(amax) * il;
             const float qs = amax > 1e-30f ? 32767.0f / amax : 0.0f;  // (a row this small stores zeros: no inf scale)
             const float f = il * qs;
-            if (lg == 0) part_ml[prow] = make_float4(m[rt], lt, qs > 0.0f ? amax * (1.0f / 32767.0f) : 0.0f, 0.0f);
-            PfPartO* dst = part_o + prow * (HD / 4) + lg;
+            if (eg == 0 && (VIA_LDS ? r < nrows : qpos[rt] >= 0))
+                part_ml[prow] = make_float4(m[rt], lt, qs > 0.0f ? amax * (1.0f / 32767.0f) : 0.0f, 0.0f);
+            if constexpr (VIA_LDS) {
 #pragma unroll
-            for (int dt = 0; dt < 16; dt++)
-                dst[4 * dt] = pack16x4(o[rt][dt][0] * f, o[rt][dt][1] * f, o[rt][dt][2] * f, o[rt][dt][3] * f);
+                for (int dt = 0; dt < 16; dt++)
+                    xch[64 * ei + ((4 * dt + eg) ^ (4 * ei))] =
+                        pack16x4(o[rt][dt][0] * f, o[rt][dt][1] * f, o[rt][dt][2] * f, o[rt][dt][3] * f);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the area is the wave's own)
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const int xr = 2 * k + (el >> 5), ro = wrow0 + 16 * rt + xr;
+                    const uint4 w = *reinterpret_cast<const uint4*>(&xch[64 * xr + ((2 * (el & 31)) ^ (4 * xr))]);
+                    const size_t orow = (size_t)sp * ps + (ro / GRP) * NH + g * GRP + ro % GRP;
+                    if (ro < nrows) *reinterpret_cast<uint4*>(part_o + orow * (HD / 4) + 2 * (el & 31)) = w;
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            } else if (qpos[rt] >= 0) {
+                PfPartO* dst = part_o + prow * (HD / 4) + eg;
+#pragma unroll
+                for (int dt = 0; dt < 16; dt++)
+                    dst[4 * dt] = pack16x4(o[rt][dt][0] * f, o[rt][dt][1] * f, o[rt][dt][2] * f, o[rt][dt][3] * f);
+            }
         }
     }  // segments
     prof_end(prof);
@@ -833,11 +863,11 @@ static void launch_prefill_pass(const float* qp, const qwa_kv_layer& kv, int nb,
     QWA_LAUNCH_MAIN(ps, (k_prefill<KVT, IMG, N>), grid, dim3(PF_THREADS), st, qp, kv, nb, p0, w.img, w.tiles, \
                     w.o, w.ml, NH * nb, upw, ns)
     if constexpr (IMG) {
-        if (nrb <= PF_FEW) QWA_PF_LAUNCH(0);
-        else if (ns == 5) QWA_PF_LAUNCH(5);
+        if (ns == 5) QWA_PF_LAUNCH(5);
         else if (ns == 6) QWA_PF_LAUNCH(6);
         else if (ns == 7) QWA_PF_LAUNCH(7);
-        else QWA_PF_LAUNCH(PF_NS);
+        else if (ns == 8) QWA_PF_LAUNCH(8);
+        else QWA_PF_LAUNCH(0);
     } else {
         QWA_PF_LAUNCH(0);
     }
