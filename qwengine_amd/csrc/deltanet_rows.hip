@@ -4,6 +4,9 @@
 // Three launches: k_dn_conv_prep (token-parallel: conv, unit q / k, and every coefficient of the chunked recurrence that
 // does not need the state), k_dn_chunk_rows (the sequential chunks of 16 tokens, on fp32 MFMA) and k_dn_gnorm_rows (the
 // gated norm to fp16).
+#include <type_traits>
+#include <utility>
+
 #include "deltanet.hpp"
 
 namespace qwa {
@@ -125,7 +128,8 @@ __global__ void __launch_bounds__(256) k_dn_conv_prep(const float* __restrict__ 
         float y[DN_CR];
         dn_conv_run<DN_CR>(qkv, cs_old, cs_new, *reinterpret_cast<const float4*>(conv_w + (size_t)c * 4), c, t0, B, y);
         __syncthreads();
-        float* dst = r.v + ((size_t)(t0 / DN_CT) * DN_VH + hv) * DN_BLK + col / 16 * 256 + col % 16 * 4 + t0 % DN_CT * 16;
+        float* dst =
+            r.v + ((size_t)(t0 / DN_CT) * DN_VH + hv) * DN_BLK + col / 16 * 256 + col % 16 * 4 + t0 % DN_CT * 16;
 #pragma unroll
         for (int u = 0; u < DN_CR; u += 4) {
             float x[4];
@@ -250,18 +254,25 @@ __global__ void __launch_bounds__(256) k_dn_conv_prep(const float* __restrict__ 
 // + 31 of its 128 x 32 slice of S (two 16-column tiles) in fp32 MFMA accumulators.  A chunk is matrix products on
 // v_mfma_f32_16x16x4_f32, per wave:
 //   a = K S (16 MFMAs, partial over the wave's key dims), summed through LDS behind the chunk's one barrier;
-//   b = Q S (16, under the latency of that exchange);
+//   b = Q S (16, mostly under the latency of that exchange);
 //   U = T W (8, in every wave: it is the operand of the wave's own update);  S = gamma_15 S + K^T (E U) (16);
 //   O = gamma b + M' U: each wave adds the product over its quarter of the tokens s (s mod 4 = w: 2) to its own partial
 //   gamma b (gamma_t scales q_t, and c2_t k_t, before the products) and leaves the sum in LDS, where the next chunk's
 //   barrier makes it visible; the threads then add the four waves' partials and store.
 // All operands come straight from global memory (L2) into registers in lane order, two chunks ahead; nothing is staged
 // through LDS.
-// What bounds it: one wave's in-order issue of 58 MFMAs (33 cycles each: 55 us for 64 chunks at 2.24 GHz) and of the
-// VALU and LDS instructions between them, on 192 of the 256 CUs.  Measured for 1024 tokens: 96 us (92 with the loads of
-// the main loop removed).  Before: 16 columns per workgroup (384 workgroups, half of the CUs with two), the operands
+// What bounds it: one wave's in-order issue, on 192 of the 256 CUs: 58 MFMAs (33 cycles each: 55 us for 64 chunks at 2.24
+// GHz) and about 28 load, store and LDS instructions per chunk, which take some 50 cycles of issue each, as the CU's four
+// waves reach them together.  Measured for 1024 tokens: 93 us.  With compiler-ordered groups of loads and 64-bit lane
+// addresses: 96 us.  Before: 16 columns per workgroup (384 workgroups, half of the CUs with two), the operands
 // staged and transposed through LDS by all threads and O in every wave: 131 us.  This kernel with the operands in row
 // order (26 load instructions per chunk instead of 12): 104 us; with 8 waves of one column tile each: 108 us.
+
+// f(0), f(1), ... with each index a compile-time constant
+template <class F, int... S>
+__device__ __forceinline__ void static_steps(F&& f, std::integer_sequence<int, S...>) {
+    (f(std::integral_constant<int, S>{}), ...);
+}
 
 // one chunk's operands of one lane
 struct DnOps {
@@ -295,174 +306,172 @@ __global__ void __launch_bounds__(DN_CW * 64, 1) k_dn_chunk_rows(DnRows r, float
     // operand addresses: a uniform chunk base and lane offsets that never change
     const uint32_t ol = 16 * l, oT = (l16 * DN_CT + 4 * g4) * 4, oE = 16 * g4, og = 8 * l16;
     const size_t kofs = (size_t)kh * DN_BLK + 512 * w, vofs = (size_t)h * DN_BLK + 512 * grp;
-    auto ld4 = [](const float* base, uint32_t off) {
-        return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(base) + off);
+    // (buffer loads: scalar base, 32-bit lane offset; a 64-bit address per lane takes twice as long to issue)
+    auto rsrc = [](const float* p, int bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, bytes, 0x00027000);
     };
-    // the loads of a chunk in four parts, issued between the MFMAs of the chunk two before it
-    auto fetch = [&](DnOps& x, int c, int part) {
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+    auto ld4 = [&](const float* base, uint32_t off) {
+        const u4v v = __builtin_amdgcn_raw_buffer_load_b128(rsrc(base, 1024), off, 0, 0);
+        return __builtin_bit_cast(float4, v);
+    };
+    // load i of a chunk's 12
+    constexpr int NLOAD = 12;
+    auto fetch = [&](DnOps& x, int c, int i) {
         const size_t kc = (size_t)c * (DN_KH * DN_BLK) + kofs;
-        if (part == 0) {
-#pragma unroll
-            for (int m = 0; m < 2; m++) x.k[m] = ld4(r.k + kc + 256 * m, ol);
-            x.T = ld4(r.coef + ((size_t)c * DN_VH + h) * DN_NCOEF, oT);
-        } else if (part == 1) {
-            const float* cf = r.coef + ((size_t)c * DN_VH + h) * DN_NCOEF;
-            x.cg = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(cf + DN_CG) + og);
-            x.E = ld4(cf + DN_CE, oE);
-            x.M = ld4(cf + DN_CM, oT);
-        } else if (part == 2) {
-#pragma unroll
-            for (int m = 0; m < 2; m++) x.q[m] = ld4(r.q + kc + 256 * m, ol);
-#pragma unroll
-            for (int n = 0; n < DN_RN; n++) x.v[n] = ld4(r.v + (size_t)c * (DN_VH * DN_BLK) + vofs + 256 * n, ol);
-        } else {
-#pragma unroll
-            for (int m = 0; m < 2; m++) x.kt[m] = ld4(r.kt + kc + 256 * m, ol);
-        }
+        const float* cf = r.coef + ((size_t)c * DN_VH + h) * DN_NCOEF;
+        if (i < 2) x.k[i] = ld4(r.k + kc + 256 * i, ol);
+        else if (i == 2)
+            x.cg = __builtin_bit_cast(float2, (u2v)__builtin_amdgcn_raw_buffer_load_b64(rsrc(cf + DN_CG, 128), og, 0, 0));
+        else if (i < 5) x.q[i - 3] = ld4(r.q + kc + 256 * (i - 3), ol);
+        else if (i < 7) x.v[i - 5] = ld4(r.v + (size_t)c * (DN_VH * DN_BLK) + vofs + 256 * (i - 5), ol);
+        else if (i == 7) x.T = ld4(cf, oT);
+        else if (i == 8) x.E = ld4(cf + DN_CE, oE);
+        else if (i < 11) x.kt[i - 9] = ld4(r.kt + kc + 256 * (i - 9), ol);
+        else x.M = ld4(cf + DN_CM, oT);
+    };
+    // c2_t k_t and gamma_t q_t: quarter i of a loaded chunk's 16 values
+    auto scale = [&](DnOps& x, int i) {
+        float4& z = i < 2 ? x.k[i & 1] : x.q[i & 1];
+        const float f = i < 2 ? x.cg.x : x.cg.y;
+        z = make_float4(f * z.x, f * z.y, f * z.z, f * z.w);
     };
     // sums the waves' partial O of chunk c: thread (wave w, lane l) the rows 4 g4 + 2 (w / 2) + {0, 1} of column tile
-    // w % 2.  Every token of the chunk is below B except in the last one
+    // w % 2 (every token of a chunk is below B except in the last one)
     const int en = w & 1, eh = w >> 1;
     float* const cobase = core_out + (size_t)(4 * g4 + 2 * eh) * DN_VD + h * DN_HD + j + 16 * en;
-    auto emit = [&](int c, bool last) {
-        float2 o = reinterpret_cast<const float2*>(&s_o[c & 1][0][en][l])[eh];
+    float2 eo[DN_CW];
+    auto emit_read = [&](int c) {
 #pragma unroll
-        for (int x = 1; x < DN_CW; x++) {
-            const float2 y = reinterpret_cast<const float2*>(&s_o[c & 1][x][en][l])[eh];
-            o.x += y.x;
-            o.y += y.y;
-        }
-        const int tok = c * DN_CT + 4 * g4 + 2 * eh;
-        float* co = cobase + (size_t)c * (DN_CT * DN_VD);
-        if (!last || tok < B) co[0] = o.x * oscale;
-        if (!last || tok + 1 < B) co[DN_VD] = o.y * oscale;
+        for (int x = 0; x < DN_CW; x++) eo[x] = reinterpret_cast<const float2*>(&s_o[c & 1][x][en][l])[eh];
     };
-    // One chunk.  A wave issues in order and its own VALU, LDS and load instructions only cost nothing between MFMAs,
-    // so the order below is fixed by scheduling barriers (DN_SB): the partial sums of a, the output of the chunk before
-    // and the fetch of chunk cf into y run between the MFMAs of b, U and the update.
+    auto emit_sum = [&]() {
+        eo[0].x = (((eo[0].x + eo[1].x) + eo[2].x) + eo[3].x) * oscale;
+        eo[0].y = (((eo[0].y + eo[1].y) + eo[2].y) + eo[3].y) * oscale;
+    };
+    float* co = cobase;  // rows of the chunk being stored
+    f4 o[DN_RN];         // partial O of the last chunk
+    // One chunk on x; z: the next chunk's operands (in registers since the chunk before), y: those of chunk cf, fetched.
+    // A wave issues in order, and its own VALU instructions cost nothing only in the shadow of an MFMA (32 cycles), so the
+    // order is fixed by a scheduling barrier (DN_SB) after every MFMA and the few instructions that go with it.
 #define DN_SB __builtin_amdgcn_sched_barrier(0)
-    auto chunk = [&](DnOps& x, int c, DnOps& y, int cf) {
+    auto chunk = [&](DnOps& x, int c, DnOps& z, DnOps& y, int cf, auto first) {
+        constexpr bool FIRST = decltype(first)::value;
         const int p = c & 1;
         f4 pa[DN_RN], pb[DN_RN], U[DN_RN];
 #pragma unroll
         for (int n = 0; n < DN_RN; n++) pa[n] = pb[n] = U[n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        const float c2 = x.cg.x, gm = x.cg.y;
-        const float g15 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gm), DN_CT - 1));
-        float kx[2][4], qx[2][4];  // c2_t k_t and gamma_t q_t
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            kx[m][0] = c2 * x.k[m].x; kx[m][1] = c2 * x.k[m].y; kx[m][2] = c2 * x.k[m].z; kx[m][3] = c2 * x.k[m].w;
-            qx[m][0] = gm * x.q[m].x; qx[m][1] = gm * x.q[m].y; qx[m][2] = gm * x.q[m].z; qx[m][3] = gm * x.q[m].w;
-        }
+        const float kx[2][4] = {{x.k[0].x, x.k[0].y, x.k[0].z, x.k[0].w}, {x.k[1].x, x.k[1].y, x.k[1].z, x.k[1].w}};
+        const float qx[2][4] = {{x.q[0].x, x.q[0].y, x.q[0].z, x.q[0].w}, {x.q[1].x, x.q[1].y, x.q[1].z, x.q[1].w}};
         const float Tx[4] = {x.T.x, x.T.y, x.T.z, x.T.w}, Ex[4] = {x.E.x, x.E.y, x.E.z, x.E.w};
-        const float ktx[2][4] = {{x.kt[0].x, x.kt[0].y, x.kt[0].z, x.kt[0].w}, {x.kt[1].x, x.kt[1].y, x.kt[1].z, x.kt[1].w}};
-        auto b_step = [&](int i) {  // MFMAs of b: reduction step i of 8, both column tiles
-#pragma unroll
-            for (int n = 0; n < DN_RN; n++) pb[n] = mfma4f32(qx[i >> 2][i & 3], st[n][i >> 2][i & 3], pb[n]);
-        };
-#pragma unroll
-        for (int n = 0; n < DN_RN; n++) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) pa[n] = mfma4f32(kx[i >> 2][i & 3], st[n][i >> 2][i & 3], pa[n]);
+        const float Mx[4] = {x.M.x, x.M.y, x.M.z, x.M.w};
+        const float ktx[2][4] = {{x.kt[0].x, x.kt[0].y, x.kt[0].z, x.kt[0].w},
+                                 {x.kt[1].x, x.kt[1].y, x.kt[1].z, x.kt[1].w}};
+        const float vx[2][4] = {{x.v[0].x, x.v[0].y, x.v[0].z, x.v[0].w}, {x.v[1].x, x.v[1].y, x.v[1].z, x.v[1].w}};
+        auto b_mfma = [&](int i, int n) { pb[n] = mfma4f32(qx[i >> 2][i & 3], st[n][i >> 2][i & 3], pb[n]); };
+        // a, the partial O of the chunk before to LDS
+        static_steps([&](auto step) __attribute__((always_inline)) {
+            constexpr int s = step.value, n = s >> 3, i = s & 7;
+            pa[n] = mfma4f32(kx[i >> 2][i & 3], st[n][i >> 2][i & 3], pa[n]);
+            if constexpr (!FIRST && (s == 2 || s == 3))
+                s_o[p ^ 1][w][s - 2][l] = make_float4(o[s - 2][0], o[s - 2][1], o[s - 2][2], o[s - 2][3]);
+            if constexpr (s == 11) s_a[p][w][0][l] = make_float4(pa[0][0], pa[0][1], pa[0][2], pa[0][3]);
+            if constexpr (s == 5 || s == 8 || s == 14) fetch(y, cf, s == 5 ? 0 : s == 8 ? 1 : 2);
             DN_SB;
-        }
-        s_a[p][w][0][l] = make_float4(pa[0][0], pa[0][1], pa[0][2], pa[0][3]);
-        b_step(0);  // under the latency of a's last MFMAs
+        }, std::make_integer_sequence<int, 16>{});
+        b_mfma(0, 0);
+        DN_SB;
+        b_mfma(0, 1);
         DN_SB;
         s_a[p][w][1][l] = make_float4(pa[1][0], pa[1][1], pa[1][2], pa[1][3]);
         __syncthreads();
-        DN_SB;
         float4 ap[DN_RN][DN_CW];
 #pragma unroll
         for (int n = 0; n < DN_RN; n++)
 #pragma unroll
             for (int v = 0; v < DN_CW; v++) ap[n][v] = s_a[p][v][n][l];
         DN_SB;
-        b_step(1);
-        b_step(2);
-        DN_SB;
-        if (c > 0) emit(c - 1, false);
-        DN_SB;
-        b_step(3);
-        b_step(4);
-        DN_SB;
-        float W[DN_RN][4];
-#pragma unroll
-        for (int n = 0; n < DN_RN; n++) {
-            const float as[4] = {((ap[n][0].x + ap[n][1].x) + ap[n][2].x) + ap[n][3].x,
-                                 ((ap[n][0].y + ap[n][1].y) + ap[n][2].y) + ap[n][3].y,
-                                 ((ap[n][0].z + ap[n][1].z) + ap[n][2].z) + ap[n][3].z,
-                                 ((ap[n][0].w + ap[n][1].w) + ap[n][2].w) + ap[n][3].w};
-            W[n][0] = x.v[n].x - as[0]; W[n][1] = x.v[n].y - as[1];
-            W[n][2] = x.v[n].z - as[2]; W[n][3] = x.v[n].w - as[3];
-            DN_SB;
-            b_step(5 + n);
-            DN_SB;
-        }
+        float W[DN_RN][4], eu[DN_RN][4];
+        uint32_t mw = 0, uw[DN_RN] = {0, 0};  // M'[l16][4 g4 + w], U[n][w]
+        const float g15 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x.cg.y), DN_CT - 1));
         f4 sn[DN_RN][2];
+        static_steps([&](auto step) __attribute__((always_inline)) {
+            constexpr int s = step.value;
+            // the rest of b, U, then per column tile the update and O
+            if constexpr (s < 14) b_mfma(1 + (s >> 1), s & 1);
+            else if constexpr (s < 22) {
+                constexpr int n = (s - 14) >> 2, e = (s - 14) & 3;
+                U[n] = mfma4f32(Tx[e], W[n][e], U[n]);
+            }
+            else {
+                constexpr int n = (s - 22) / 9, k = (s - 22) % 9;
+                if constexpr (k < 8) sn[n][k & 1] = mfma4f32(ktx[k & 1][k >> 1], eu[n][k >> 1], sn[n][k & 1]);
+                else o[n] = mfma4f32(__uint_as_float(mw), __uint_as_float(uw[n]), pb[n]);
+            }
+            if constexpr (!FIRST) {  // the output of the chunk before
+                if constexpr (s == 14) emit_read(c - 1);
+                if constexpr (s == 25) emit_sum();
+                if constexpr (s == 27) co[0] = eo[0].x;
+                if constexpr (s == 30) co[DN_VD] = eo[0].y;
+            }
+            if constexpr (s >= 6 && s < 14) {  // W = beta v - a
+                constexpr int n = (s - 6) >> 2, e = (s - 6) & 3;
+                auto at = [&](int v) {
+                    return e == 0 ? ap[n][v].x : e == 1 ? ap[n][v].y : e == 2 ? ap[n][v].z : ap[n][v].w;
+                };
+                W[n][e] = vx[n][e] - (((at(0) + at(1)) + at(2)) + at(3));
+            }
+            if constexpr (s >= 14 && s < 18) sn[(s - 14) >> 1][s & 1] = st[(s - 14) >> 1][s & 1] * g15;
+            if constexpr (s == 20 || s == 24) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) eu[(s - 20) >> 2][e] = Ex[e] * U[(s - 20) >> 2][e];
+            }
+            if constexpr (s == 2) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) mw |= __float_as_uint(Mx[e]) & wm[e];
+            }
+            if constexpr (s == 26 || s == 28) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) uw[(s - 26) >> 1] |= __float_as_uint(U[(s - 26) >> 1][e]) & wm[e];
+            }
+            if constexpr (s >= 34 && s < 38) scale(z, s - 34);
+            if constexpr (s % 4 == 1 && s / 4 < NLOAD - 3) fetch(y, cf, 3 + s / 4);
+            DN_SB;
+        }, std::make_integer_sequence<int, 40>{});
+        if constexpr (!FIRST) co += DN_CT * DN_VD;
 #pragma unroll
         for (int n = 0; n < DN_RN; n++)
 #pragma unroll
-            for (int m = 0; m < 2; m++) sn[n][m] = st[n][m] * g15;
-        DN_SB;
-        b_step(7);
-        DN_SB;
-#pragma unroll
-        for (int n = 0; n < DN_RN; n++) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) U[n] = mfma4f32(Tx[e], W[n][e], U[n]);
-            DN_SB;
-            fetch(y, cf, n);
-            DN_SB;
-        }
-        f4 o[DN_RN];
-        const uint32_t mw = (__float_as_uint(x.M.x) & wm[0]) | (__float_as_uint(x.M.y) & wm[1]) |
-                            (__float_as_uint(x.M.z) & wm[2]) | (__float_as_uint(x.M.w) & wm[3]);  // M'[l16][4 g4 + w]
-#pragma unroll
-        for (int n = 0; n < DN_RN; n++) {
-            float eu[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) eu[e] = Ex[e] * U[n][e];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-#pragma unroll
-                for (int m = 0; m < 2; m++) sn[n][m] = mfma4f32(ktx[m][e], eu[e], sn[n][m]);
-                if (e == 1) {
-                    DN_SB;
-                    fetch(y, cf, 2 + n);
-                    DN_SB;
-                }
-            }
-            uint32_t uw = 0;  // U[n][w]
-#pragma unroll
-            for (int e = 0; e < 4; e++) uw |= __float_as_uint(U[n][e]) & wm[e];
-            o[n] = mfma4f32(__uint_as_float(mw), __uint_as_float(uw), pb[n]);
-            DN_SB;
-        }
-#pragma unroll
-        for (int n = 0; n < DN_RN; n++) {
-            s_o[p][w][n][l] = make_float4(o[n][0], o[n][1], o[n][2], o[n][3]);
-#pragma unroll
             for (int m = 0; m < 2; m++) st[n][m] = sn[n][m];
-        }
     };
     // two chunks ahead, three register sets; every fetch is unconditional (past the end: the last chunk again) so that
     // the compiler can count the loads in flight and waits for no later ones
     DnOps xa, xb, xc;
 #pragma unroll
-    for (int part = 0; part < 4; part++) fetch(xa, 0, part);
+    for (int i = 0; i < NLOAD; i++) fetch(xa, 0, i);
 #pragma unroll
-    for (int part = 0; part < 4; part++) fetch(xb, min(1, nch - 1), part);
-    int c = 0;
+    for (int i = 0; i < NLOAD; i++) fetch(xb, min(1, nch - 1), i);
+#pragma unroll
+    for (int i = 0; i < 4; i++) scale(xa, i);
+    const int last = nch - 1;
+    chunk(xa, 0, xb, xc, min(2, last), std::true_type{});
+    int c = 1;
     for (; c + 3 <= nch; c += 3) {
-        chunk(xa, c, xc, c + 2);
-        chunk(xb, c + 1, xa, min(c + 3, nch - 1));
-        chunk(xc, c + 2, xb, min(c + 4, nch - 1));
+        chunk(xb, c, xc, xa, min(c + 2, last), std::false_type{});
+        chunk(xc, c + 1, xa, xb, min(c + 3, last), std::false_type{});
+        chunk(xa, c + 2, xb, xc, min(c + 4, last), std::false_type{});
     }
-    if (c < nch) chunk(xa, c, xc, nch - 1);
-    if (c + 1 < nch) chunk(xb, c + 1, xa, nch - 1);
+    if (c < nch) chunk(xb, c, xc, xa, last, std::false_type{});
+    if (c + 1 < nch) chunk(xc, c + 1, xa, xb, last, std::false_type{});
+#pragma unroll
+    for (int n = 0; n < DN_RN; n++) s_o[last & 1][w][n][l] = make_float4(o[n][0], o[n][1], o[n][2], o[n][3]);
     __syncthreads();
-    emit(nch - 1, true);
+    emit_read(last);
+    emit_sum();
+    const int tok = last * DN_CT + 4 * g4 + 2 * eh;
+    if (tok < B) co[0] = eo[0].x;
+    if (tok + 1 < B) co[DN_VD] = eo[0].y;
 #pragma unroll
     for (int n = 0; n < DN_RN; n++)
 #pragma unroll
@@ -504,8 +513,8 @@ hipError_t launch_dn_rows(const qwa_dn_params& p, const float* qkv, const float*
     const float* cs_old = p.conv_state + (size_t)cin * 3 * DN_CH;
     float* cs_new = p.conv_state + (size_t)(cin ^ 1) * 3 * DN_CH;
     const int runs = nch * (DN_CT / DN_CR);
-    hipLaunchKernelGGL(k_dn_conv_prep, dim3(DN_KH * nch + DN_VD / 256 * runs), dim3(256), 0, st, qkv, cs_old, p.conv_w, r,
-                       beta_raw, alpha_raw, p.dt_bias, p.ssm_a, eps, B, nch, cs_new);
+    hipLaunchKernelGGL(k_dn_conv_prep, dim3(DN_KH * nch + DN_VD / 256 * runs), dim3(256), 0, st, qkv, cs_old, p.conv_w,
+                       r, beta_raw, alpha_raw, p.dt_bias, p.ssm_a, eps, B, nch, cs_new);
     hipLaunchKernelGGL(k_dn_chunk_rows, dim3(DN_VH, DN_RG), dim3(DN_CW * 64), 0, st, r, p.ssm_state, B, core_out);
     hipLaunchKernelGGL(k_dn_gnorm_rows, dim3(B), dim3(256), 0, st, core_out, z, p.ssm_norm, eps, o16);
     return hipGetLastError();
