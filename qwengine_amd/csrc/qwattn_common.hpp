@@ -76,21 +76,34 @@ __device__ __forceinline__ float wave_sum(float v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+// lane moves inside a row of 16 lanes (DPP, no LDS round trip): quad_perm [1,0,3,2] and [2,3,0,1], row_half_mirror (lane i
+// <-> 7 - i) and row_mirror (i <-> 15 - i), which meet the lanes at distance 4 and 8 once quads and octets agree
+template <int CTRL>
+__device__ __forceinline__ float row_move(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
 }
-// reductions over the 32-lane half of a wave that holds one quant block
-__device__ __forceinline__ float half_sum(float v) {
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 32);
-    return v;
-}
+// reductions over the 32-lane half of a wave that holds one quant block: the maximum, and the sum of whole numbers below
+// 2^24 (both exact in any order); every lane of the half active
 __device__ __forceinline__ float half_max(float v) {
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 32));
-    return v;
+    v = fmaxf(v, row_move<0xB1>(v));
+    v = fmaxf(v, row_move<0x4E>(v));
+    v = fmaxf(v, row_move<0x141>(v));
+    v = fmaxf(v, row_move<0x140>(v));
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+__device__ __forceinline__ float half_sum(float v) {
+    v += row_move<0xB1>(v);
+    v += row_move<0x4E>(v);
+    v += row_move<0x141>(v);
+    v += row_move<0x140>(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+__device__ __forceinline__ float wave_max(float v) {
+    v = half_max(v);
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
