@@ -65,10 +65,10 @@ __device__ __forceinline__ void put8(float* p, const float* x) {
     }
 }
 
-// reductions over the 4 lanes of one quant block / the 32 lanes of one half
+// maximum over the 4 lanes of one quant block
 __device__ __forceinline__ float quad_max(float v) {
-    v = fmaxf(v, __shfl_xor(v, 1, 64));
-    return fmaxf(v, __shfl_xor(v, 2, 64));
+    v = fmaxf(v, row_move<0xB1>(v));
+    return fmaxf(v, row_move<0x4E>(v));
 }
 
 // Quantize the 256-value row held by one half (lane l of the half owns elements 8l..8l+7) into the split layout.
@@ -182,9 +182,7 @@ __device__ __forceinline__ void rms_norm_half(float* x, const float* w, int l, f
     float ss = 0.0f;
 #pragma unroll
     for (int j = 0; j < VPL; j++) ss += x[j] * x[j];
-#pragma unroll
-    for (int o = 1; o < 32; o <<= 1) ss += __shfl_xor(ss, o, 64);
-    const float r = rsqrtf(ss / (float)HD + eps);
+    const float r = rsqrtf(half_sum(ss) / (float)HD + eps);
     float wv[VPL];
     load8(w + VPL * l, wv);
 #pragma unroll
@@ -287,29 +285,11 @@ __global__ void __launch_bounds__(256) k_prep_rows(const float* qg, const float*
 // of gates.
 // What bounds it: the bytes (111 MB for 1024 tokens, 22 us at the card's copy rate).  Measured there, Q8_0, with the rope
 // table's launch: 23.9 us (k_prep_rows: 47.7); the kernel alone 21.8 us (45.4 before).
-template <int CTRL>
-__device__ __forceinline__ float kv_dpp(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
-}
-// sum over the 32 lanes of a half: lane distances 1, 2, 4, 8, 16 (the mirrored lane of an 8- or 16-lane group holds the
-// same value as the lane at distance 4 or 8 once the lanes of the group's quads, or octets, agree)
-__device__ __forceinline__ float half_sum32(float v) {
-    v += kv_dpp<0xB1>(v);
-    v += kv_dpp<0x4E>(v);
-    v += kv_dpp<0x141>(v);
-    v += kv_dpp<0x140>(v);
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
-}
 // the value of the lane 4 further (lanes 0-3 of a row) or 4 back (lanes 4-7)
 __device__ __forceinline__ float xor4_low(float x) {
     const int v = __float_as_int(x);
     const int up = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xF, 0x1, true);                 // row_shl:4 into bank 0
     return __int_as_float(__builtin_amdgcn_update_dpp(up, v, 0x114, 0xF, 0x2, false));       // row_shr:4 into bank 1
-}
-__device__ __forceinline__ float quad_max_dpp(float v) {
-    v = fmaxf(v, kv_dpp<0xB1>(v));
-    return fmaxf(v, kv_dpp<0x4E>(v));
 }
 
 // quant_row for aligned rows: x[0..7] = elements 8 l .. 8 l + 7 of the half's row
@@ -326,7 +306,7 @@ __device__ __forceinline__ void quant_row_al(uint8_t* vals, uint16_t* scales, co
             float a = 0.0f;
 #pragma unroll
             for (int j = 0; j < VPL; j++) a = fmaxf(a, fabsf(x[j]));
-            d = quad_max_dpp(a) / 127.0f;
+            d = quad_max(a) / 127.0f;
             const float id = d != 0.0f ? 1.0f / d : 0.0f;
             uint32_t w[2] = {0u, 0u};
 #pragma unroll
@@ -346,8 +326,8 @@ __device__ __forceinline__ void quant_row_al(uint8_t* vals, uint16_t* scales, co
                 mx = t ? om : mx;
                 ix = t ? oi : ix;
             };
-            take(kv_dpp<0xB1>(am), kv_dpp<0xB1>(mx), __builtin_amdgcn_update_dpp(0, ix, 0xB1, 0xF, 0xF, true));
-            take(kv_dpp<0x4E>(am), kv_dpp<0x4E>(mx), __builtin_amdgcn_update_dpp(0, ix, 0x4E, 0xF, 0xF, true));
+            take(row_move<0xB1>(am), row_move<0xB1>(mx), __builtin_amdgcn_update_dpp(0, ix, 0xB1, 0xF, 0xF, true));
+            take(row_move<0x4E>(am), row_move<0x4E>(mx), __builtin_amdgcn_update_dpp(0, ix, 0x4E, 0xF, 0xF, true));
             d = mx / -8.0f;
             const float id = d != 0.0f ? 1.0f / d : 0.0f;
             uint32_t w = 0u;
@@ -403,7 +383,7 @@ __global__ void __launch_bounds__(256) k_prep_rows_al(const float* __restrict__ 
         float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < VPL; j++) ss += x[j] * x[j];
-        const float rs = rsqrtf(half_sum32(ss) / (float)HD + eps);
+        const float rs = rsqrtf(half_sum(ss) / (float)HD + eps);
 #pragma unroll
         for (int j = 0; j < VPL; j++) x[j] = x[j] * rs * wv[j];
 #pragma unroll
