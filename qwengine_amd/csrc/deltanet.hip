@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(DN_HT) k_dn_head(qwa_dn_params p, int cin, qwa
         const int tt = t >> 7, i = t0 + tt;
         const bool emit = tt < nt && i >= n_commit;
         const float y0 = s_o[tt][jn];
-        const float ss = wave_sum(y0 * y0);
+        const float ss = wave_sum_sq_low(y0);
         if (lane == 0) s_red[tt][wave & 1] = ss;
         __syncthreads();
         if (emit) {

@@ -45,8 +45,8 @@ __host__ __device__ inline DnRows dn_rows_split(void* work, int nch) {
     return r;
 }
 
-// 13056 floats per token; the size asked for is never below 14432 per token + 33792 per chunk, which callers may have
-// reserved for a longer call
+// `need`: 14400 floats per token of the padded chunks + the coefficients.  The size asked for is never below `least` (the
+// conv, q / k and gate rows in token order), which callers may have reserved for a longer call
 size_t dn_work_bytes(int B) {
     const size_t nch = (B + DN_CT - 1) / DN_CT;
     const size_t need = nch * (DN_BLK * (DN_VH + 3 * DN_KH) + DN_VH * DN_NCOEF);

@@ -77,9 +77,9 @@ template <int CTRL>
 __device__ __forceinline__ float row_move(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
 }
-// reductions over the 32-lane half of a wave that holds one quant block, and over the wave: lane distances 1, 2, 4, 8, 16,
-// 32.  (A sum over the wave through LDS permutes is six dependent round trips: with them the GEMV at 6144 -> 5120 took
-// 7.05 us instead of 6.9 for one column, IQ3_S 15.8 instead of 12.4 for four.)
+// reductions over the 32-lane half of a wave that holds one quant block, and over the wave.  (A sum over the wave through
+// LDS permutes is six dependent round trips: with them the GEMV at 6144 -> 5120 took 7.05 us instead of 6.9 for one
+// column, IQ3_S 15.8 instead of 12.4 for four.)
 __device__ __forceinline__ float half_max(float v) {
     v = fmaxf(v, row_move<0xB1>(v));
     v = fmaxf(v, row_move<0x4E>(v));
@@ -101,11 +101,25 @@ __device__ __forceinline__ float wave_max(float v) {
     const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }
-
+// sums: lane distances 32, 16, 8, 4, 2, 1, a fixed tree, as codes are quantized from what it feeds.  (A rotation of a row
+// by 8 or 4, 0x128 and 0x124, meets the lane at that distance: all of a row for 8, and for 4 once the lanes 8 apart agree.)
+__device__ __forceinline__ float half_tree(float v) {
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    v += row_move<0x128>(v);
+    v += row_move<0x124>(v);
+    v += row_move<0x4E>(v);
+    return v + row_move<0xB1>(v);
+}
 __device__ __forceinline__ float wave_sum(float v) {
-    v = half_sum(v);
     const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    return half_tree(__uint_as_float(a[0]) + __uint_as_float(a[1]));
+}
+// sum of y * y in lanes 0 .. 31, the first step as one FMA: y^2 of lane i + 32 rounded, that of lane i not
+__device__ __forceinline__ float wave_sum_sq_low(float y) {
+    const uint32_t p = __float_as_uint(y * y);
+    const auto a = __builtin_amdgcn_permlane32_swap(p, p, false, false);
+    return half_tree(fmaf(y, y, __uint_as_float(a[1])));
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
