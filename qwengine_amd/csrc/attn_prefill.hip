@@ -25,79 +25,16 @@
 
 #include "kv_operands.hpp"
 #include "launch.hpp"
+#include "pf_plan.hpp"
 
 namespace qwa {
 
 #ifndef QWA_PF_XCD
 #define QWA_PF_XCD 1
 #endif
-#ifndef QWA_PF_WAVES
-#define QWA_PF_WAVES 8
-#endif
-constexpr int PF_WAVES = QWA_PF_WAVES;           // MFMA waves per workgroup
 constexpr int PF_THREADS = PF_WAVES * 64;
 constexpr int PF_WPE = PF_WAVES / 4;             // waves per SIMD
-#ifndef QWA_PF_RT
-#define QWA_PF_RT (16 / PF_WAVES > 0 ? 16 / PF_WAVES : 1)
-#endif
-constexpr int PF_RT = QWA_PF_RT;                 // 16-row MFMA tiles per wave
-constexpr int PF_ROWS = PF_WAVES * PF_RT * 16;   // rows per workgroup
-constexpr int PF_TILE = 32;                      // keys per tile
 constexpr int PF_KT = PF_TILE / 16;              // 16-key MFMA tiles per tile
-constexpr int PF_NS = PF_ROWS == 192 ? 6 : 8;    // key-range splits per row block (3 rounds of the chip for B = 1024)
-constexpr int PF_MAXB = 1024;                    // tokens per pass
-// row blocks of a pass of nb tokens (per KV head)
-inline int pf_row_blocks(int nb) { return (GRP * nb + PF_ROWS - 1) / PF_ROWS; }
-constexpr int PF_FEW = 12;  // row blocks up to which a pass takes the split count that fills one round of the chip
-// splits of a pass of nb tokens whose keys end at npos.
-// Up to PF_FEW row blocks (512 tokens): as many as make one round of the 256 CUs (64 / row blocks per KV head), each of
-// at least one tile.  (Fewer splits for short key ranges, sqrt(c tiles / tokens) with c = 500 .. 2000 to weigh the
-// partial states, measured the same or up to 3 us slower at contexts below 4000.)
-// Measured, whole call, us, against 5 to 8 splits for every pass (Q8_0): 8 tokens at 20000 positions 153 -> 48, 77 at
-// 20011 167 -> 84, 77 at 90000 648 -> 281, 128 at 32256 255 -> 152, 200 at 5000 69 -> 60, 256 at 32256 261 -> 235;
-// 512 tokens unchanged (their 5 splits already make one round).
-// Above that (at most PF_NS): the count that fills the chip's 256 CUs in whole rounds best, i.e. the fewest rounds per
-// split, ceil(workgroups / 256) / splits (1024 tokens: 8 splits, 3 rounds).
-inline int pf_splits(int nb, int npos) {
-    const int nrb = pf_row_blocks(nb);
-    if (nrb <= PF_FEW) return min(256 / (NKV * nrb), (npos - 1) / PF_TILE + 1);
-    const int groups = nrb * NKV;
-    int best = PF_NS;
-    for (int ns = PF_NS - 1; ns >= 5; ns--)  // 5 .. PF_NS: the instantiated kernels
-        if ((long)((groups * ns + 255) / 256) * best < (long)((groups * best + 255) / 256) * ns) best = ns;
-    return best;
-}
-// Whether a call dequantises its KV range into fp16 images first.  The image pass and the wider fp16 stream pay when
-// several row blocks read a tile; up to these counts every workgroup converts its raw tiles in the loop instead.
-// Whole call, us, images / raw tiles: F16 42 tokens at 60000 positions 166 / 100, 77 at 20011 92 / 76, 170 at 20000
-// (4 blocks) 127 / 122, 256 at 32256 (6) 243 / 253; Q4_0 150 / 105, 84 / 80, 120 / 128 (4 blocks); Q8_0 150 / 129,
-// 84 / 88, 122 / 144.
-inline bool pf_use_image(int kvt, int nb) {
-    return pf_row_blocks(nb) > (kvt == QWA_KV_F16 ? 4 : kvt == QWA_KV_Q4_0 ? 2 : 1);
-}
-// token-splits (splits x tokens) that a workspace for passes of up to nb tokens has to hold: PF_NS per token, or what
-// the shorter passes take (at most 256 / NKV / row blocks splits each: 2736 token-splits cover every count of row
-// blocks), never decreasing in nb
-inline int pf_token_splits(int nb) { return max(PF_NS * nb, min(256 / NKV * nb, 2736)); }
-#ifndef QWA_PF_UPW
-#define QWA_PF_UPW 1
-#endif
-#ifndef QWA_PF_SEG_MAXPOS
-#define QWA_PF_SEG_MAXPOS 81920
-#endif
-// (row block, KV head, split) units per workgroup of a pass of nb tokens whose keys end at npos: as many as make the
-// units one round of the chip's 256 CUs, when the split count is 8 (so the workgroups of one XCD walk the splits in
-// step, see k_prefill) and the pass's keys end within QWA_PF_SEG_MAXPOS; otherwise 1, the units running in rounds.
-// Measured, whole call, 1024 tokens (in-process A/B against rounds): Q8_0 -31 us at p0 = 0, -30 at 8192, -43 at
-// 32768, -43 at 49152, -23 at 65536, +19 at 100000 (Q4_0 -48 at 32768, -12 at 100000; F16 -41 at 32768).  Past
-// ~80000 positions a workgroup's three splits are long enough for the row blocks sharing an XCD's L2 to drift apart.
-// (QWA_PF_UPW = 0: always rounds.)
-inline int pf_units_per_wg(int nb, int npos) {
-    const int nrb = pf_row_blocks(nb), ns = pf_splits(nb, npos);
-    if (!QWA_PF_UPW || nrb <= PF_FEW || ns != 8 || npos > QWA_PF_SEG_MAXPOS) return 1;
-    const int units = nrb * NKV * ns;
-    return (units + 255) / 256;
-}
 constexpr int KS_LD = HD + 8;                    // K tile row stride (halves)
 constexpr int VT_LD = PF_TILE + 8;               // V^T tile row stride (halves)
 #ifndef QWA_PF_VD
@@ -291,9 +228,6 @@ __device__ __forceinline__ void pf_convert(const uint8_t* raw, _Float16* Ks, _Fl
     }
 }
 
-constexpr int PF_IMG_K = PF_TILE * HD * 2;      // bytes of the K part of an image: [32 keys][256 dims] fp16
-constexpr int PF_IMG_BYTES = 2 * PF_IMG_K;      // K part, then V^T part [256 dims][32 keys] fp16
-constexpr int PF_IMG_NBUF = 3;   // images in LDS: the one computed on and two in flight
 constexpr int PF_IMG_AHEAD = 2;
 
 // Image layout (unpadded, so that a direct-to-LDS copy of 1 KB per instruction reproduces it in LDS, and XOR-swizzled
@@ -686,12 +620,12 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
         // 509 tokens at 0 F16 39.7 -> 36.2, 77 at 20011 Q8_0 87.7 -> 82.7, 256 at 32256 242.8 -> 240.1; the 1024-token
         // kernel (8 splits), whose one store per 400 tiles does not matter, measured 774 -> 778 and stores directly, as do
         // the raw-tile kernels, whose ring is too small
-        constexpr bool VIA_LDS = IMG && NS != 8;
+        constexpr bool VIA_LDS = IMG && NS != 8 && PF_XCH_FITS;
         // (an opaque copy of the lane: the addresses below must not live across the key loop)
         int el = lane;
         if constexpr (VIA_LDS) asm volatile("" : "+v"(el));
         const int ei = VIA_LDS ? el & 15 : i16, eg = VIA_LDS ? el >> 4 : lg;
-        uint2* const xch = reinterpret_cast<uint2*>(&s_raw[0][0]) + wave * 1024;
+        uint2* const xch = reinterpret_cast<uint2*>(&s_raw[0][0]) + wave * (PF_XCH_BYTES / 8);
         if constexpr (VIA_LDS) __syncthreads();  // no wave's images are in flight any more
 #pragma unroll
         for (int rt = 0; rt < PF_RT; rt++) {
