@@ -511,15 +511,20 @@ __device__ __forceinline__ void dq_sub(const uint8_t* b, int j, float* v, const 
     }
 }
 
-// A workgroup decodes DQ_RUNS runs of 256 consecutive sub-blocks (consecutive in W and in out, across rows), a thread
-// one sub-block of each run, with one expansion of the codebook.  A thread's 64 output bytes would go out as four stores
-// that each touch every second 128-byte line of the wave's 4 KB; they change lanes in LDS instead (16-byte units, XOR-
-// swizzled against bank conflicts), so that every store instruction writes one contiguous 1 KB.
-// What bounds it: the bytes (63 MB written, 8 to 14 MB read for 5120 x 6144: 14 us at the card's copy rate).  Measured at
-// that size, us, one sub-block per thread with direct stores / this: IQ3_S 23.6 / 15.3, IQ2_XS 23.5 / 14.5, IQ2_XXS
-// 22.9 / 14.0, IQ2_S 25.5 / 15.4, Q4_K 23.2 / 15.1, Q6_K 26.6 / 21.8.
-constexpr int DQ_RUNS = 4;
-template <int FMT>
+// A workgroup decodes RUNS runs of 256 consecutive sub-blocks (consecutive in W and in out, across rows), a thread one
+// sub-block of each run, with one expansion of the codebook.  A thread's 64 output bytes would go out as four stores that
+// each touch every second 128-byte line of the wave's 4 KB; they change lanes in LDS instead (16-byte units, XOR-swizzled
+// against bank conflicts), so that every store instruction writes one contiguous 1 KB.
+// What bounds it: the bytes (5120 x 6144: 63 MB written and 8 to 26 read).  Measured at that size with weights and output
+// that no cache holds, us, direct stores / this: Q2_K 26.5 / 17.0, Q4_K 27.4 / 18.4, Q6_K 30.5 / 20.3, IQ4_XS 27.5 / 18.2,
+// IQ2_XXS 25.8 / 17.6, IQ2_XS 27.4 / 19.0, IQ2_S 29.7 / 21.0, IQ3_XXS 26.9 / 17.6, IQ3_S 28.0 / 18.1.
+// One run: more runs are a serial chain in each workgroup, which shows most where the call leaves the chip idle (four
+// runs, 16 to 256 rows of 6144: 5.6-7.0 us instead of 3.3-4.1; 5120 rows: 20.1-23.0 instead of 17.5-20.3).  IQ2_S alone,
+// whose codebook and sign masks (11 KB) take as long to expand as a run to decode, does two once the call fills the chip
+// anyway (DQ_PAIRED sub-blocks: 1536 rows of 5120 7.7 us with one run, 7.6 with two; 5120 rows 15.0 / 13.6; below, 64
+// rows 4.2 / 4.9).
+constexpr long long DQ_PAIRED = 4 * 256 * 256;
+template <int FMT, int RUNS>
 __global__ void __launch_bounds__(256) k_dequant_f16(const uint8_t* __restrict__ W, size_t row_bytes, int K, int rows,
                                                      uint16_t* __restrict__ out) {
     const uint32_t nsub = (uint32_t)K / 32;
@@ -529,11 +534,11 @@ __global__ void __launch_bounds__(256) k_dequant_f16(const uint8_t* __restrict__
         WFmt<FMT>::fill(s_grid, threadIdx.x, 256);
         __syncthreads();
     }
-    const long long total = (long long)rows * nsub, first = (long long)blockIdx.x * (256 * DQ_RUNS);
+    const long long total = (long long)rows * nsub, first = (long long)blockIdx.x * (256 * RUNS);
     const int row0 = (int)(first / nsub), lane = threadIdx.x & 63;  // (uniform: one division per workgroup)
     const uint32_t rem0 = (uint32_t)(first - (long long)row0 * nsub);
     uint4* const buf = s_out[threadIdx.x >> 6];
-    for (int run = 0; run < DQ_RUNS; run++) {
+    for (int run = 0; run < RUNS; run++) {
         const long long wave_i = first + 256 * run + (threadIdx.x & ~63u);  // the wave's first sub-block
         if (wave_i >= total) return;
         const uint32_t at = rem0 + 256 * run + threadIdx.x;
@@ -560,8 +565,10 @@ __global__ void __launch_bounds__(256) k_dequant_f16(const uint8_t* __restrict__
             const uint4 q = buf[(x & ~3) | ((x & 3) ^ ((x >> 3) & 3))];
             if (x < units) dst[x] = q;
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        if (RUNS > 1) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
     }
 }
 
@@ -661,17 +668,23 @@ hipError_t launch_dequant_f16(int fmt, const void* W, size_t rb, int K, int rows
         return hipGetLastError();
     }
     const long long n = (long long)rows * (K / 32);
-    const dim3 grid((unsigned)((n + 256 * DQ_RUNS - 1) / (256 * DQ_RUNS))), block(256);
+    auto launch = [&](auto kernel, int runs) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((n + 256 * runs - 1) / (256 * runs))), dim3(256), 0, st, w, rb, K, rows,
+                           out);
+    };
     switch (fmt) {
-        case QWA_W_Q2_K: hipLaunchKernelGGL(k_dequant_f16<QWA_W_Q2_K>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_Q4_K: hipLaunchKernelGGL(k_dequant_f16<QWA_W_Q4_K>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_Q6_K: hipLaunchKernelGGL(k_dequant_f16<QWA_W_Q6_K>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_IQ4_XS: hipLaunchKernelGGL(k_dequant_f16<QWA_W_IQ4_XS>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_IQ2_XXS: hipLaunchKernelGGL(k_dequant_f16<QWA_W_IQ2_XXS>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_IQ2_XS: hipLaunchKernelGGL(k_dequant_f16<QWA_W_IQ2_XS>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_IQ2_S: hipLaunchKernelGGL(k_dequant_f16<QWA_W_IQ2_S>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_IQ3_XXS: hipLaunchKernelGGL(k_dequant_f16<QWA_W_IQ3_XXS>, grid, block, 0, st, w, rb, K, rows, out); break;
-        case QWA_W_IQ3_S: hipLaunchKernelGGL(k_dequant_f16<QWA_W_IQ3_S>, grid, block, 0, st, w, rb, K, rows, out); break;
+        case QWA_W_Q2_K: launch(k_dequant_f16<QWA_W_Q2_K, 1>, 1); break;
+        case QWA_W_Q4_K: launch(k_dequant_f16<QWA_W_Q4_K, 1>, 1); break;
+        case QWA_W_Q6_K: launch(k_dequant_f16<QWA_W_Q6_K, 1>, 1); break;
+        case QWA_W_IQ4_XS: launch(k_dequant_f16<QWA_W_IQ4_XS, 1>, 1); break;
+        case QWA_W_IQ2_XXS: launch(k_dequant_f16<QWA_W_IQ2_XXS, 1>, 1); break;
+        case QWA_W_IQ2_XS: launch(k_dequant_f16<QWA_W_IQ2_XS, 1>, 1); break;
+        case QWA_W_IQ2_S:
+            if (n >= DQ_PAIRED) launch(k_dequant_f16<QWA_W_IQ2_S, 2>, 2);
+            else launch(k_dequant_f16<QWA_W_IQ2_S, 1>, 1);
+            break;
+        case QWA_W_IQ3_XXS: launch(k_dequant_f16<QWA_W_IQ3_XXS, 1>, 1); break;
+        case QWA_W_IQ3_S: launch(k_dequant_f16<QWA_W_IQ3_S, 1>, 1); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

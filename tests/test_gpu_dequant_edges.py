@@ -1,5 +1,5 @@
-"""Prefill dequantizer at the edges of its work split (waves of 64 sub-blocks, runs of 256, workgroups of 1024; rows shorter
-and longer than a wave's span, row strides wider than the row): bit-exact with the oracle's fp32 value rounded to fp16
+"""Prefill dequantizer at the edges of its work split (waves of 64 sub-blocks, workgroups of 256, or of two runs of 256 in
+large IQ2_S calls; rows shorter and longer than a wave's span, row strides wider than the row): bit-exact with the oracle's fp32 value rounded to fp16
 (nearest-even), and nothing written behind the output."""
 import numpy as np
 import pytest
@@ -25,3 +25,10 @@ def test_dequant_edges_bit_exact(gpu, oracle, fmt, K, rows, pad):
     want = oracle.w_dequant(fmt, Wn, K).astype(np.float16).reshape(-1)
     assert np.array_equal(out[:rows * K].cpu().numpy().view(np.uint16), want.view(np.uint16))
     assert torch.isnan(out[rows * K:]).all()
+
+
+@pytest.mark.parametrize("K,rows", [(256, 32767), (256, 32768), (256, 32801), (256, 32833), (2304, 3641)])
+def test_dequant_iq2_s_paired_runs(gpu, oracle, K, rows):
+    """IQ2_S from 262144 sub-blocks on: two runs a workgroup; the last workgroup full, ending in its first run, in its
+    second one, and across rows."""
+    test_dequant_edges_bit_exact(gpu, oracle, ops.W_IQ2_S, K, rows, 0)
