@@ -335,13 +335,13 @@ template <int FMT> struct GvBatched {
         QWA_GV_BATCH >= 0 ? QWA_GV_BATCH == 1 : FMT != QWA_W_IQ4_XS && FMT != QWA_W_Q2_K && FMT != QWA_W_Q6_K;
 };
 
-// One wave per row; NB activation columns at aq + c * act_ld (d / s at + c * act_ld / 32)
-template <int FMT, int NB, int U>
-__global__ void __launch_bounds__(GV_WAVES * 64) k_gemv_q8(const uint8_t* __restrict__ W, size_t row_bytes, int K,
-                                                           int N, const int8_t* __restrict__ aq,
-                                                           const float* __restrict__ ad, const float* __restrict__ as,
-                                                           int act_ld, float* __restrict__ y, int y_ld,
-                                                           int accumulate) {
+// One wave per row; NB activation columns at aq + c * act_ld (d / s at + c * act_ld / 32).
+// WPE: 0, or the waves per SIMD that the registers are given out for (see gv_narrow).
+template <int FMT, int NB, int U, int WPE = 0>
+__global__ void __launch_bounds__(GV_WAVES * 64) __attribute__((amdgpu_waves_per_eu(WPE ? 4 : 2, WPE ? WPE : 8)))
+k_gemv_q8(const uint8_t* __restrict__ W, size_t row_bytes, int K, int N, const int8_t* __restrict__ aq,
+          const float* __restrict__ ad, const float* __restrict__ as, int act_ld, float* __restrict__ y, int y_ld,
+          int accumulate) {
     using F = WFmt<FMT>;
     const int lane = threadIdx.x & 63;
     const int nsub = K / 32;
@@ -602,18 +602,49 @@ bool gemv_q8_supported(int fmt) {
            fmt == QWA_W_IQ2_XS || fmt == QWA_W_IQ2_S || fmt == QWA_W_IQ3_XXS || fmt == QWA_W_IQ3_S;
 }
 
+// The narrow form of a kernel: registers for at most this many waves per SIMD, so that the compiler keeps more of a row's
+// loads in flight; 0: none.  A kernel of 8-wave workgroups keeps 2 of them on a CU then, where the wide form has 3 (or 4).
+// The wide form wins where that makes the grid one round instead of two, the narrow one where its third workgroup has no
+// use: see gv_narrow.  The forms listed are those whose wide form was slower than the same kernel with its sums through LDS
+// permutes, which had taken more registers for them.
+// Measured, us, K = 17408, LDS permutes / wide / narrow: four columns IQ4_XS 1000 rows 13.7 / 14.1 / 9.4, 5120 34.7 /
+// 26.9 / 30.2, 8000 39.3 / 47.0 / 41.2; Q2_K 36.6 / 42.8 / 36.3 at 8000; IQ3_S 45.6 / 48.7 / 41.9 at 8000; three columns
+// IQ4_XS 10.8 / 13.2 / 10.3 at 2000, Q4_K 32.3 / 33.6 / 29.1 at 8000; two columns IQ2_XXS 7.7 / 9.0 / 7.6 at 1000 (at
+// K = 5120 the wide form is the faster one); one column Q4_K 8.8 / 8.8 / 7.4 at 1000, 26.3 / 27.6 / 24.9 at 8000.
+constexpr int gv_narrow_waves(int fmt, int nb, int u) {
+    const bool plain = fmt == QWA_W_Q2_K || fmt == QWA_W_Q4_K || fmt == QWA_W_Q6_K || fmt == QWA_W_IQ4_XS;
+    if (nb == 4) return fmt == QWA_W_Q4_K ? 0 : 5;
+    if (nb == 3) return plain ? 6 : 0;
+    if (nb == 2) return plain ? 0 : 6;
+    return fmt == QWA_W_Q4_K && u == 4 ? 5 : 0;
+}
+// Whether a call of `groups` workgroups takes it: up to 2 workgroups per CU (1 with two columns, whose chain per sub-block
+// is short), and again past one round of 3 per CU.  Two columns: only for rows past 8192, five or more sub-blocks a lane.
+inline bool gv_narrow(int nb, int groups, int K) {
+    return (groups <= (nb == 2 ? 256 : 512) || groups > 768) && (nb != 2 || K > 8192);
+}
+
 template <int FMT>
 static hipError_t gemv_fmt(const void* W, size_t rb, int K, int N, const qwa_act_q8& a, int nb, int act_ld, float* y,
                            int y_ld, int acc, hipStream_t st) {
-    const dim3 grid((unsigned)min((N + GV_WAVES - 1) / GV_WAVES, 65535)), block(GV_WAVES * 64);
+    const int groups = min((N + GV_WAVES - 1) / GV_WAVES, 65535);
     const uint8_t* w = static_cast<const uint8_t*>(W);
     // one column: a lane's sub-block rounds (K / 2048 of them, up to 4) loaded as one batch, for the formats whose
     // decode chain is long enough to gain from it (measured: Q4_K and the grid formats; IQ4_XS, Q2_K, Q6_K run
     // faster one sub-block at a time).  Several columns keep one sub-block per batch (registers).
     const int rounds = (K / 32 + 63) / 64;
     const int ub = (nb == 1 && GvBatched<FMT>::value) ? min(rounds, 4) : 1;
-#define QWA_GV_LAUNCH(NB, U) \
-    hipLaunchKernelGGL((k_gemv_q8<FMT, NB, U>), grid, block, 0, st, w, rb, K, N, a.q, a.d, a.s, act_ld, y, y_ld, acc)
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(GV_WAVES * 64), 0, st, w, rb, K, N, a.q, a.d, a.s, act_ld, y,
+                           y_ld, acc);
+    };
+    const bool narrow = gv_narrow(nb, groups, K);
+#define QWA_GV_LAUNCH(NB, U)                                         \
+    do {                                                             \
+        constexpr int WPE = gv_narrow_waves(FMT, NB, U);             \
+        if (WPE != 0 && narrow) run(k_gemv_q8<FMT, NB, U, WPE>);     \
+        else run(k_gemv_q8<FMT, NB, U>);                             \
+    } while (0)
     switch (nb) {
         case 1:
             switch (ub) {
