@@ -811,7 +811,7 @@ static void launch_prefill_pass(const float* qp, const qwa_kv_layer& kv, int nb,
 hipError_t launch_prefill(const float* q, const float* gate, const qwa_kv_layer& kv, int kvt, int B, int p0,
                           uint16_t* out16, void* work, hipStream_t st) {
     const PfWork w = pf_work_layout(static_cast<uint8_t*>(work), B, p0 + B);
-    const bool image = pf_use_image(kvt, min(B, PF_MAXB));
+    const bool image = pf_use_image(kvt, min(B, PF_MAXB), p0 + B);
     if (image) {
         const dim3 grid(w.tiles, NKV);
         if (kvt == QWA_KV_F16)

@@ -42,13 +42,26 @@ constexpr int pf_splits(int nb, int npos) {
         if ((long)((groups * ns + 255) / 256) * best < (long)((groups * best + 255) / 256) * ns) best = ns;
     return best;
 }
-// Whether a call dequantises its KV range into fp16 images first.  The image pass and the wider fp16 stream pay when
-// several row blocks read a tile; up to these counts every workgroup converts its raw tiles in the loop instead.
-// Whole call, us, images / raw tiles: F16 42 tokens at 60000 positions 166 / 100, 77 at 20011 92 / 76, 170 at 20000
-// (4 blocks) 127 / 122, 256 at 32256 (6) 243 / 253; Q4_0 150 / 105, 84 / 80, 120 / 128 (4 blocks); Q8_0 150 / 129,
-// 84 / 88, 122 / 144.
-constexpr bool pf_use_image(int kvt, int nb) {
-    return pf_row_blocks(nb) > (kvt == QWA_KV_F16 ? 4 : kvt == QWA_KV_Q4_0 ? 2 : 1);
+// Whether a call of nb tokens whose keys end at npos dequantises its KV range into fp16 images first (the results are the
+// same bits either way).  Otherwise every workgroup converts its raw tiles in the loop: once more per row block, slower to
+// start (a workgroup's first tile is converted before anything runs) and with 32-byte stores of its partial states, but
+// without the image pass's launch and its 64 KB written and read per tile.  So the raw tiles win for the fewest row blocks
+// and, with more of them, only from some length of the key range on; the cheaper the conversion, the earlier (F16: a copy).
+// Whole call, us, images / raw tiles.  F16: 8 tokens at 200 positions 22.5 / 19.6, 36 at 0 23.6 / 24.4 and at 1500 34.6 /
+// 34.4; 42 (1 block) at 2000 34.8 / 35.5, at 3500 38.3 / 37.4, at 60000 163 / 113; 64 (2) at 3200 39.1 / 39.9, at 5000
+// 42.9 / 42.4, at 20000 83.7 / 73.2; 110 (3) at 5000 49.1 / 49.3, at 8192 60.5 / 59.4, at 20000 105 / 97; 150 (4) at 14336
+// 93.8 / 94.5, at 20000 120 / 116; 171 (5) at 20000 140 / 144.  Q4_0: 8 at 200 24.6 / 21.9, 36 at 1500 39.6 / 38.9; 42 (1)
+// at 2500 40.7 / 42.3, at 6500 47.0 / 46.4, at 60000 139 / 112; 64 (2) at 14336 67.8 / 68.3, at 20000 80.8 / 79.7, at 60000
+// 182 / 171; 110 (3) at 60000 233 / 243.  Q8_0: 8 at 200 22.6 / 21.6, 20 at 1000 28.7 / 29.3 and at 3500 36.3 / 35.1; 42
+// (1) at 2000 34.7 / 38.4, at 16384 60.1 / 60.0, at 60000 147 / 132; 64 (2) at 60000 188 / 196.
+constexpr bool pf_use_image(int kvt, int nb, int npos) {
+    constexpr int MAX_BLOCKS = 4, NEVER = MAX_POS + 1;
+    const int nrb = pf_row_blocks(nb);
+    if (nb <= (kvt == QWA_KV_Q8_0 ? 20 : 36)) return false;
+    if (nrb > MAX_BLOCKS) return true;
+    constexpr int f16[MAX_BLOCKS] = {2560, 4096, 6144, 16384}, q4[MAX_BLOCKS] = {4608, 18432, NEVER, NEVER},
+                  q8[MAX_BLOCKS] = {16384, NEVER, NEVER, NEVER};
+    return npos < (kvt == QWA_KV_F16 ? f16 : kvt == QWA_KV_Q4_0 ? q4 : q8)[nrb - 1];
 }
 // the most token-splits (splits x tokens) that a pass of up to PF_FEW row blocks takes (2728 of 256 rows, at 341 tokens)
 constexpr int pf_few_token_splits() {

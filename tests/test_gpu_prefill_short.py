@@ -36,6 +36,30 @@ def test_short_pass_vs_oracle(gpu, oracle, cache, B, p0):
     assert_close(out.float().cpu().numpy(), ref, f"B={B} p0={p0}")
 
 
+# either side of every line between raw tiles and images: tokens, and positions for 1, 2, 3, 4 row blocks
+ROUTES = {ops.F16: [(36, 900), (37, 900), (42, 2559), (42, 2560), (85, 4095), (85, 4096), (128, 6143), (128, 6144),
+                    (170, 16383), (170, 16384), (171, 16384)],
+          ops.Q8_0: [(20, 900), (21, 900), (42, 16383), (42, 16384), (43, 16384)],
+          ops.Q4_0: [(36, 900), (37, 900), (42, 4607), (42, 4608), (85, 18431), (85, 18432), (86, 18432)]}
+
+
+@pytest.mark.parametrize("kvt", KVTS, ids=lambda k: KV_NAMES[k])
+def test_both_forms_at_the_lines_between_them(gpu, oracle, kvt):
+    kv, _, _ = make_cache(kvt, 18432, 18432, seed=930 + kvt)
+    Kd, Vd = dequant_cache(kv, 18432)
+    for B, n in ROUTES[kvt]:
+        print(f"prefill form {KV_NAMES[kvt]} B={B} n={n}", flush=True)
+        q, gate = seeded_normal((B, 24, 256), 940 + B), seeded_normal((B, 24, 256), 941 + B)
+        out = torch.full((B, 24, 256), float("nan"), dtype=torch.float16, device="cuda")
+        work = torch.full((ops.attn_prefill_work_bytes(B, n) // 4,), float("nan"), device="cuda")
+        ops.attn_prefill_ws(q, gate, kv, kvt, B, n - B, out, work)
+        torch.cuda.synchronize()
+        # the oracle on the first, a middle and the last tokens
+        for t in (0, B // 2, B - 3):
+            ref = oracle.attention(q[t:t + 3].cpu().numpy(), gate[t:t + 3].cpu().numpy(), Kd, Vd, n - B + t, 3)
+            assert_close(out[t:t + 3].float().cpu().numpy(), ref, f"B={B} n={n} t={t}")
+
+
 def test_work_bytes_never_decrease(gpu):
     """A workspace for a longer chunk or context covers every shorter call."""
     for n in (1, 33, 5000, 262144):
