@@ -619,7 +619,7 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
         // that a store instruction writes two whole 512-byte rows instead of 32-byte pieces of 16 rows.  Whole call, us:
         // 509 tokens at 0 F16 39.7 -> 36.2, 77 at 20011 Q8_0 87.7 -> 82.7, 256 at 32256 242.8 -> 240.1; the 1024-token
         // kernel (8 splits), whose one store per 400 tiles does not matter, measured 774 -> 778 and stores directly, as do
-        // the raw-tile kernels, whose ring is too small
+        // the raw-tile kernels, whose ring is too small (their fp16 tiles would hold it; not measured)
         constexpr bool VIA_LDS = IMG && NS != 8 && PF_XCH_FITS;
         // (an opaque copy of the lane: the addresses below must not live across the key loop)
         int el = lane;
@@ -796,11 +796,14 @@ static void launch_prefill_pass(const float* qp, const qwa_kv_layer& kv, int nb,
 #define QWA_PF_LAUNCH(N)                                                                                              \
     QWA_LAUNCH_MAIN(ps, (k_prefill<KVT, IMG, N>), grid, dim3(PF_THREADS), st, qp, kv, nb, p0, w.img, w.tiles, \
                     w.o, w.ml, NH * nb, upw, ns)
+    // 8 splits: the kernel of the long passes stores its partial states directly, which the few tiles per split of a short
+    // pass do not pay for (same bits, whole call, us, that kernel / the general one: 320 tokens at 0 Q8_0 36.7 / 33.5, at
+    // 5000 77.0 / 73.0, at 20000 191 / 185, at 60000 493 / 486); with 5 to 7 splits the compiled counts are 0 to 3% faster
     if constexpr (IMG) {
         if (ns == 5) QWA_PF_LAUNCH(5);
         else if (ns == 6) QWA_PF_LAUNCH(6);
         else if (ns == 7) QWA_PF_LAUNCH(7);
-        else if (ns == 8) QWA_PF_LAUNCH(8);
+        else if (ns == 8 && nrb > PF_FEW) QWA_PF_LAUNCH(8);
         else QWA_PF_LAUNCH(0);
     } else {
         QWA_PF_LAUNCH(0);

@@ -30,7 +30,11 @@ constexpr int PF_FEW = 12;  // row blocks up to which a pass takes the split cou
 // partial states, measured the same or up to 3 us slower at contexts below 4000.)
 // Measured, whole call, us, against 5 to 8 splits for every pass (Q8_0): 8 tokens at 20000 positions 153 -> 48, 77 at
 // 20011 167 -> 84, 77 at 90000 648 -> 281, 128 at 32256 255 -> 152, 200 at 5000 69 -> 60, 256 at 32256 261 -> 235;
-// 512 tokens unchanged (their 5 splits already make one round).
+// 512 tokens unchanged (their 5 splits already make one round).  Odd counts, too: the next lower even one would let
+// k_prefill number the row blocks that share a tile onto one XCD, but its longer splits cost more than that gives (whole
+// call, us, the count / the even one: 21 / 20 splits, 128 tokens at 20000 F16 positions 99.5 / 102.5, Q8_0 103.1 / 103.0,
+// at 149000 576 / 591; 9 / 8, 298 at 20000 174 / 178, at 149000 1067 / 1112; 7 / 6, 384 at 60000 551 / 595; 5 / 4, 512 at
+// 60000 716 / 841).
 // Above that (at most PF_NS): the count that fills the chip's 256 CUs in whole rounds best, i.e. the fewest rounds per
 // split, ceil(workgroups / 256) / splits (1024 tokens: 8 splits, 3 rounds).
 constexpr int pf_splits(int nb, int npos) {

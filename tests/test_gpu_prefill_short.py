@@ -36,6 +36,13 @@ def test_short_pass_vs_oracle(gpu, oracle, cache, B, p0):
     assert_close(out.float().cpu().numpy(), ref, f"B={B} p0={p0}")
 
 
+@pytest.mark.parametrize("B,p0", [(86, 139), (86, 170), (299, 0), (320, 41), (341, 5700)])
+def test_short_pass_of_eight_splits(gpu, oracle, cache, B, p0):
+    """8 splits, by the row blocks (299 to 341 tokens) or by the tiles (keys that end at 225 to 256): not the kernel of the
+    1024-token passes, which have as many."""
+    test_short_pass_vs_oracle(gpu, oracle, cache, B, p0)
+
+
 # either side of every line between raw tiles and images: tokens, and positions for 1, 2, 3, 4 row blocks
 ROUTES = {ops.F16: [(36, 900), (37, 900), (42, 2559), (42, 2560), (85, 4095), (85, 4096), (128, 6143), (128, 6144),
                     (170, 16383), (170, 16384), (171, 16384)],
