@@ -850,7 +850,7 @@ hipError_t launch_prefill(const float* q, const float* gate, const qwa_kv_layer&
         switch (ns) {
 #define QWA_PF_COMBINE(N) \
     case N: hipLaunchKernelGGL(k_pf_combine<N>, cg, cb, 0, st, gp, nrows, w.o, w.ml, nrows, upw, op); break
-            QWA_PF_COMBINE(5); QWA_PF_COMBINE(6); QWA_PF_COMBINE(7);
+            QWA_PF_COMBINE(6); QWA_PF_COMBINE(7);
             default: hipLaunchKernelGGL(k_pf_combine<PF_NS>, cg, cb, 0, st, gp, nrows, w.o, w.ml, nrows, upw, op); break;
 #undef QWA_PF_COMBINE
         }

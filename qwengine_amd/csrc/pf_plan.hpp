@@ -42,7 +42,7 @@ constexpr int pf_splits(int nb, int npos) {
     if (nrb <= PF_FEW) return std::min(256 / (NKV * nrb), (npos - 1) / PF_TILE + 1);
     const int groups = nrb * NKV;
     int best = PF_NS;
-    for (int ns = PF_NS - 1; ns >= 5; ns--)  // 5 .. PF_NS: the instantiated kernels
+    for (int ns = PF_NS - 1; ns >= 6; ns--)  // 6 .. PF_NS: 5 splits are never the best of these passes
         if ((long)((groups * ns + 255) / 256) * best < (long)((groups * best + 255) / 256) * ns) best = ns;
     return best;
 }

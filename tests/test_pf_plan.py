@@ -46,3 +46,14 @@ def test_workspace_holds_every_pass(tmp_path, waves, rt):
                     "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_longer_passes_take_the_instantiated_split_counts(tmp_path):
+    """Past 12 row blocks: 6, 7 or 8 splits, each of them by some pass (the combine is built for these)."""
+    src, exe = tmp_path / "plan.cpp", tmp_path / "plan"
+    src.write_text('#include <stdio.h>\n#include "pf_plan.hpp"\nint main() { for (int nb = 513; nb <= 1024; nb++) '
+                   'printf("%d ", qwa::pf_splits(nb, 262144)); }')
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "qwengine_amd", "csrc"), "-I",
+                    os.path.join(ROOT, "include"), str(src), "-o", str(exe)], check=True)
+    counts = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()
+    assert set(counts) == {"6", "7", "8"}
