@@ -178,10 +178,12 @@ def _ptr(t) -> int | None:
 
 def _stream(stream) -> int | None:
     if stream is None:
-        if not torch.cuda.is_initialized():  # (with no GPU context yet, current_stream creates it)
-            return torch.cuda.current_stream().cuda_stream if torch.cuda.is_available() else None
         # the current stream's handle without building a Stream object, which costs 3 us, a quarter of a short decode call
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+        if raw is not None and device is not None and torch.cuda.is_initialized():
+            return raw(device())
+        # (with no GPU context yet, current_stream creates it)
+        return torch.cuda.current_stream().cuda_stream if torch.cuda.is_available() else None
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
