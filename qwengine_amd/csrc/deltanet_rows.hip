@@ -45,8 +45,9 @@ __host__ __device__ inline DnRows dn_rows_split(void* work, int nch) {
     return r;
 }
 
-// `need`: 14400 floats per token of the padded chunks + the coefficients.  The size asked for is never below `least` (the
-// conv, q / k and gate rows in token order), which callers may have reserved for a longer call
+// `need`: 14400 floats per token of the padded chunks, 12288 of v, q, k and kt and 2112 of coefficients.  For whole chunks
+// the stated size stays the one that this entry point has always stated (`least`: rows in token order, no padding), with
+// nothing stored in the difference; short and ragged calls need the padding (1 token: 922 KB).
 size_t dn_work_bytes(int B) {
     const size_t nch = (B + DN_CT - 1) / DN_CT;
     const size_t need = nch * (DN_BLK * (DN_VH + 3 * DN_KH) + DN_VH * DN_NCOEF);
