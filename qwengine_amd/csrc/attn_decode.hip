@@ -1296,7 +1296,8 @@ extern template __global__ void k_dec3h<QWA_KV_F16>(const float* __restrict__, q
 // Bound by latency: one round trip for the records, one LDS exchange of the groups' sums.  Lane r of every wave holds
 // record r's (m, l), so the maximum and the factors need no exchange between the waves; a factor reaches its group's sums
 // as a scalar.  With the maximum, the factors and the sums each exchanged through LDS behind a barrier of their own, a
-// layer's call took 0.5 us more at 4096 F16 positions (13.2 -> 12.7) and 0.65 at 150000 Q4_0 (41.6 -> 40.95).
+// layer's call took 0.5 us more at 4096 F16 positions (13.2 -> 12.7); at 32775 positions and beyond the calls measured the
+// same within 1%.
 __global__ void __launch_bounds__(256) k_dec_combine(const float* __restrict__ work, int nsplit, int halves,
                                                      const float* __restrict__ gate, float* __restrict__ out,
                                                      float* __restrict__ out_host, qwa_act_q8 oq, int do_q) {
