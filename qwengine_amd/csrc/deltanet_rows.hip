@@ -95,14 +95,16 @@ __device__ __forceinline__ void dn_conv_run(const float* __restrict__ qkv, const
 
 __device__ __forceinline__ float dn_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-// One launch, two kinds of blocks of 256 threads (bound by the bytes: 42 MB read and 42 MB written for 1024 tokens).
+// One launch, two kinds of blocks of 256 threads (bound by the bytes: for 1024 tokens 42 MB read and 57 MB written, 20 us
+// at the card's copy rate).
 //  * blocks 0 .. 16 nch - 1: (key head, chunk).  Thread = channel of the key head's q | k; the conv of the chunk's 16
 //    tokens, L2 norms through LDS (unit q / k written out and kept in LDS), the Gram products k.k and q.k on fp32
 //    MFMA (each wave half of the 128 dims of one of the two), then wave v < 3 forms the coefficient block of value head
 //    kh + 16 v: L and M' from the Gram entries and the decay products, T by forward substitution (lane = column).
 //    The three value heads of a key head share the conv, the norms and the Gram products.
 //  * the rest: (256 v channels, run of 8 tokens): the conv, times the token's beta for the head.
-// Measured for 1024 tokens: 24 us (a conv kernel and a per-value-head preparation kernel before: 21 + 22 us).
+// Measured for 1024 tokens: 24 us, 21 once the clock has settled (a conv kernel and a per-value-head preparation kernel
+// before: 21 + 22 us, 18 + 20 settled).
 constexpr int DN_CR = 8;                  // tokens per run of the v channels
 constexpr int DN_XP = 2 * DN_HD + 4;      // padded row (floats) of the chunk's q | k in LDS
 __global__ void __launch_bounds__(256) k_dn_conv_prep(const float* __restrict__ qkv, const float* __restrict__ cs_old,
@@ -264,10 +266,11 @@ __global__ void __launch_bounds__(256) k_dn_conv_prep(const float* __restrict__ 
 // through LDS.
 // What bounds it: one wave's in-order issue, on 192 of the 256 CUs: 58 MFMAs (33 cycles each: 55 us for 64 chunks at 2.24
 // GHz) and about 28 load, store and LDS instructions per chunk, which take some 50 cycles of issue each, as the CU's four
-// waves reach them together.  Measured for 1024 tokens: 93 us.  With compiler-ordered groups of loads and 64-bit lane
-// addresses: 96 us.  Before: 16 columns per workgroup (384 workgroups, half of the CUs with two), the operands
-// staged and transposed through LDS by all threads and O in every wave: 131 us.  This kernel with the operands in row
-// order (26 load instructions per chunk instead of 12): 104 us; with 8 waves of one column tile each: 108 us.
+// waves reach them together.  Measured for 1024 tokens, in one session: 93 us (86 once the clock has settled); with
+// compiler-ordered groups of loads and 64-bit lane addresses: 96 us.  Before: 16 columns per workgroup (384 workgroups, half
+// of the CUs with two), the operands staged and transposed through LDS by all threads and O in every wave: 131 us.  This
+// kernel with the operands in row order (26 load instructions per chunk instead of 12): 104 us; with 8 waves of one column
+// tile each: 108 us.
 
 // f(0), f(1), ... with each index a compile-time constant
 template <class F, int... S>
