@@ -16,11 +16,12 @@
 //    accumulator already in B-operand layout; online softmax in fp32 with a lazy rescale;
 //  * the causal key range of a row block is cut into fixed splits (pf_splits) so that the 24 row blocks x 4 KV
 //    heads of a 1024-token chunk fill the chip, up to 64 of them for the one row block of a short chunk; the (row
-//    block, KV head, split) units run one per workgroup, or, for a 1024-token pass, three consecutive ones per workgroup in a single round (pf_units_per_wg), a run of splits of
-//    one row block being walked as one key range.  Each run leaves a partial state (m, l, O / l) in the caller's
-//    workspace and k_pf_combine merges them in a fixed order, applies the sigmoid gate and writes fp16.  Chunks
-//    longer than PF_MAXB tokens run as several passes.  Nothing here allocates: the images and partial states live
-//    in a workspace of prefill_work_bytes(B, p0 + B) bytes.
+//    block, KV head, split) units run one per workgroup, or, for a 1024-token pass, three consecutive ones per
+//    workgroup in a single round (pf_units_per_wg), a run of splits of one row block being walked as one key range.
+//    Each run leaves a partial state (m, l, O / l) in the caller's workspace; k_pf_combine, or k_pf_combine_any for
+//    short passes, merges them in a fixed order, applies the sigmoid gate and writes fp16.  Chunks longer than PF_MAXB
+//    tokens run as several passes.  Nothing here allocates: the images and partial states live in a workspace of
+//    prefill_work_bytes(B, p0 + B) bytes.
 #include <float.h>
 
 #include "kv_operands.hpp"
@@ -472,7 +473,8 @@ k_prefill(const float* __restrict__ q, qwa_kv_layer kv, int B, int p0, const uin
             const int k0 = (tb + i) * PF_TILE, cur = i & 1;
             // raw Q4_0 tiles: opaque copies of the thread index, so that the load's and the conversion's per-thread
             // addresses are formed anew for every tile instead of living across the loop (31 -> 18 spilled registers;
-            // 42 tokens at 60000 positions 112 -> 105 us; the other formats measured 1-5% slower this way)
+            // 42 tokens at 60000 positions 112 -> 105 us; the other formats measured 1-5% slower this way, and the raw
+            // kernels still spill: 19 registers of F16, 40 of Q8_0)
             int tl = t, ll = lane;
             if constexpr (!IMG && KVT == QWA_KV_Q4_0) asm volatile("" : "+v"(tl), "+v"(ll));
             // tile i + AHEAD (the last tile again near the end: a harmless re-read) into the raw buffer freed last
