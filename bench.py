@@ -445,7 +445,8 @@ def consumer_extras(ops, torch, steps):
         blocks[:, :, 1] = 0x1c  # every d (and Q4_K's dmin) field a small fp16 value: bytes xx 1c ~ 0.004
         if fmt == ops.W_Q4_K:
             blocks[:, :, 3] = 0x1c
-        # enough copies to pass 300 MB, so that neither the L2s nor the 256 MB MALL serve the weights
+        # distinct copies, so that the L2s do not serve the weights (a graph's 16 calls read 130 to 283 MB, which for the
+        # grid formats the 256 MB last-level cache does)
         nw = -(-300_000_000 // (N * rb))
         W = [torch.from_numpy(Wn).cuda() for _ in range(nw)]
 
