@@ -67,12 +67,15 @@ constexpr bool pf_use_image(int kvt, int nb, int npos) {
                   q8[MAX_BLOCKS] = {16384, NEVER, NEVER, NEVER};
     return npos < (kvt == QWA_KV_F16 ? f16 : kvt == QWA_KV_Q4_0 ? q4 : q8)[nrb - 1];
 }
-// the most token-splits (splits x tokens) that a pass of up to PF_FEW row blocks takes (2728 of 256 rows, at 341 tokens)
+// the most token-splits (splits x tokens) that a pass of up to PF_FEW row blocks takes (2728 of 256 rows, at 341 tokens),
+// rounded up to a multiple of 16: the partial states start behind this many (m, l) rows, and 150 tokens at 0 Q8_0 positions
+// take 29.8 us behind 2728 of them and 27.7 behind 2736 (their splits lie 1.8 MB apart, so the start decides how they share
+// the memory channels)
 constexpr int pf_few_token_splits() {
     int most = 0;
     for (int nrb = 1; nrb <= PF_FEW; nrb++)
         most = std::max(most, std::min(nrb * PF_ROWS / GRP, PF_MAXB) * (256 / (NKV * nrb)));
-    return most;
+    return (most + 15) & ~15;
 }
 // token-splits that a workspace for passes of up to nb tokens has to hold: PF_NS per token, or what the shorter passes
 // take, never decreasing in nb
